@@ -163,7 +163,11 @@ struct LuFactorArgs {
 };
 int launch_lu_factor(const LuFactorArgs &a, hipStream_t s);
 int launch_lu_solve(const double *LU, const int *piv, double *b, int n, int count, hipStream_t s);
-int launch_derivative(const double *D, int N, long long ncols, const double *u, double *out, hipStream_t s);
+// Element-wise z derivative: DT is derivative_operand(D, N) on the device;
+// derivative_prepare once per plan (the kernel's LDS limit on the current device).
+std::vector<double> derivative_operand(const std::vector<double> &D, int N);
+int derivative_prepare(int N);
+int launch_derivative(const double *DT, int N, long long ncols, const double *u, double *out, hipStream_t s);
 // Multiplies the half spectrum re/im[A][B][lanes] by (2 pi i k/len)^order along
 // axis A (axis_a) or B of length L (Fourier derivative).
 int launch_spectral_derivative(double *re, double *im, long long A, long long B, long long lanes, int axis_a, int L,
@@ -226,6 +230,8 @@ struct hz_plan {
     std::vector<double> z, Dz, Dzz, shift;
     // device
     double *d_Dz = nullptr, *d_Dzz = nullptr, *d_DzzT = nullptr, *d_shift = nullptr;
+    double *d_DzT = nullptr;  // hz_derivative_z's operands: Dz's, then (DzT_n further on) Dzz's
+    size_t DzT_n = 0;
     double2 *d_twx = nullptr, *d_twy = nullptr;
     hz::Spectrum spec, bc;
     int *d_status = nullptr;

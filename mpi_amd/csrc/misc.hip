@@ -2,34 +2,79 @@
 // SecondDerivativeZ, NonPeriodic3D_MPI.cpp:632-683).
 //
 // out[e][i][j][k] = sum_p D[k][p] u[e][i][j][p] for every element column:
-// a batch of small dense products, each thread producing one output node of
-// one column (columns are contiguous, so a wave reads and writes consecutive
-// z values; the N x N matrix stays in the caches).  The sum runs over
-// p = 0..N-1 in order with every product rounded before it is added, as in
-// the reference's loop, so the result equals the reference's bit for bit.
+// a batch of small dense products.  The sum runs over p = 0..N-1 in order
+// with every product rounded before it is added, as in the reference's loop,
+// so the result equals the reference's bit for bit.
 #include "hz_internal.h"
 
 namespace hz {
 namespace {
 
-__device__ __forceinline__ double rounded_dot(const double *__restrict__ a, const double *__restrict__ b, int n)
-{
-#pragma clang fp contract(off)
-    double acc = 0.0;
-    for (int p = 0; p < n; ++p) acc += a[p] * b[p];
-    return acc;
-}
+// Lanes are columns, a wave's registers hold kDerivRows output rows of 64
+// columns.  The column tile is staged in LDS (a lane's values one column
+// stride apart: the stride is odd, so 64 lanes hit different banks); the
+// matrix value of a step is the same in every lane, so it comes through the
+// scalar cache from the transposed copy DT[p][k] (KP = N rounded up to
+// kDerivRows).  One LDS read and kDerivRows products and sums a step, where a
+// thread per output node read a matrix row (uncoalesced) and a column from
+// the caches for every pair.  256^2 columns of N = 129: 2,727 -> 137 us; the
+// rounded products and sums cannot be fused, N^2 of each per column, which is
+// 55 us at one 16-lane operation per clock, and the rest is the scalar loads'
+// latency (the matrix, 149 KB, does not fit the scalar cache).
+constexpr int kDerivRows = 16;
+constexpr int kDerivCols = 64;
 
-__global__ __launch_bounds__(256) void derivative_kernel(const double *__restrict__ D, int N, long long ncols,
+__global__ __launch_bounds__(1024) void derivative_kernel(const double *__restrict__ DT, int N, int KP, long long ncols,
                                                          const double *__restrict__ u, double *__restrict__ out)
 {
-    const long long total = ncols * N;
-    for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        const long long col = idx / N;
-        const int k = (int)(idx % N);
-        const double *uc = u + col * N;
-        out[idx] = rounded_dot(D + (long long)k * N, uc, N);
+#pragma clang fp contract(off)
+    extern __shared__ double dtile[];
+    const int LD = N | 1;  // odd column stride
+    const long long col0 = (long long)blockIdx.x * kDerivCols;
+    const int nc = (int)(ncols - col0 < kDerivCols ? ncols - col0 : kDerivCols);
+    const double *src = u + col0 * N;
+    const int total = nc * N, T = blockDim.x;
+    if (LD == N) {
+        constexpr int U = 8;
+        int i = threadIdx.x;
+        for (; i + (U - 1) * T < total; i += U * T) {
+            double v[U];
+#pragma unroll
+            for (int j = 0; j < U; ++j) v[j] = src[i + j * T];
+#pragma unroll
+            for (int j = 0; j < U; ++j) dtile[i + j * T] = v[j];
+        }
+        for (; i < total; i += T) dtile[i] = src[i];
+    } else {
+        for (int i = threadIdx.x; i < total; i += T) dtile[i + i / N] = src[i];
+    }
+    __syncthreads();
+    const int lane = threadIdx.x % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), waves = T / 64;
+    const double *uc = dtile + (lane < nc ? lane : 0) * LD;
+    for (int k0 = wave * kDerivRows; k0 < N; k0 += waves * kDerivRows) {
+        double acc[kDerivRows];
+#pragma unroll
+        for (int j = 0; j < kDerivRows; ++j) acc[j] = 0.0;
+        const double *d = DT + k0;
+#pragma unroll 2
+        for (int p = 0; p < N; ++p) {
+            const double x = uc[p];
+#pragma unroll
+            for (int j = 0; j < kDerivRows; ++j) acc[j] += d[(long long)p * KP + j] * x;
+        }
+        if (lane < nc) {
+            double *o = out + (col0 + lane) * N + k0;
+            const int rows = N - k0 < kDerivRows ? N - k0 : kDerivRows;
+            if (rows == kDerivRows) {
+#pragma unroll
+                for (int j = 0; j < kDerivRows; ++j) o[j] = acc[j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < kDerivRows; ++j)
+                    if (j < rows) o[j] = acc[j];
+            }
+        }
     }
 }
 
@@ -176,12 +221,35 @@ int launch_cubic_adjoint(const double *fbar, const double *u_in, const double *u
     return HZ_OK;
 }
 
-int launch_derivative(const double *D, int N, long long ncols, const double *u, double *out, hipStream_t s)
+std::vector<double> derivative_operand(const std::vector<double> &D, int N)
+{
+    const int KP = (N + kDerivRows - 1) / kDerivRows * kDerivRows;
+    std::vector<double> t((size_t)N * KP, 0.0);
+    for (int k = 0; k < N; ++k)
+        for (int p = 0; p < N; ++p) t[(size_t)p * KP + k] = D[(size_t)k * N + p];
+    return t;
+}
+
+int derivative_prepare(int N)
+{
+    const size_t lds = sizeof(double) * kDerivCols * (N | 1);
+    if (lds > 64 * 1024)
+        HZ_HIP(hipFuncSetAttribute((const void *)derivative_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   160 * 1024));
+    return HZ_OK;
+}
+
+int launch_derivative(const double *DT, int N, long long ncols, const double *u, double *out, hipStream_t s)
 {
     if (ncols <= 0) return HZ_OK;
-    const long long total = ncols * N;
-    const int blocks = (int)std::min<long long>((total + 255) / 256, 4096);
-    hipLaunchKernelGGL(derivative_kernel, dim3(blocks), dim3(256), 0, s, D, N, ncols, u, out);
+    const int strips = (N + kDerivRows - 1) / kDerivRows;
+    // one strip per wave, at most 16 waves (evenly filled passes above)
+    const int passes = (strips + 15) / 16, waves = std::max(2, (strips + passes - 1) / passes);
+    const size_t lds = sizeof(double) * kDerivCols * (N | 1);
+    const long long blocks = (ncols + kDerivCols - 1) / kDerivCols;
+    if (lds > 160 * 1024 || blocks > 0x7fffffffLL) return set_error(HZ_ERR_UNSUPPORTED, "derivative: field too large");
+    hipLaunchKernelGGL(derivative_kernel, dim3((unsigned)blocks), dim3(64 * waves), (unsigned)lds, s, DT, N,
+                       strips * kDerivRows, ncols, u, out);
     HZ_HIP(hipGetLastError());
     return HZ_OK;
 }
@@ -205,5 +273,5 @@ extern "C" int hz_derivative_z(hz_plan *p, int order, const double *u, double *o
 {
     if (!p || !u || !out || (order != 1 && order != 2)) return set_error(HZ_ERR_ARG, "bad argument");
     const long long ncols = (long long)p->ne * p->nx * p->ny;
-    return launch_derivative(order == 1 ? p->d_Dz : p->d_Dzz, p->N, ncols, u, out, (hipStream_t)stream);
+    return launch_derivative(order == 1 ? p->d_DzT : p->d_DzT + p->DzT_n, p->N, ncols, u, out, (hipStream_t)stream);
 }

@@ -71,6 +71,7 @@ void free_plan(hz_plan *p)
     (void)hipFree(p->d_Dz);
     (void)hipFree(p->d_Dzz);
     (void)hipFree(p->d_DzzT);
+    (void)hipFree(p->d_DzT);
     (void)hipFree(p->d_shift);
     (void)hipFree(p->d_twx);
     (void)hipFree(p->d_twy);
@@ -937,10 +938,14 @@ int hz_plan_create(const hz_plan_desc *desc, hz_plan **plan)
     std::vector<double> DzzT((size_t)p->n * p->n);
     for (int i = 0; i < p->n; ++i)
         for (int j = 0; j < p->n; ++j) DzzT[(size_t)j * p->n + i] = p->Dzz[(size_t)(i + 1) * p->N + (j + 1)];
+    std::vector<double> DzT = derivative_operand(p->Dz, p->N);
+    p->DzT_n = DzT.size();
+    const std::vector<double> DzzTd = derivative_operand(p->Dzz, p->N);
+    DzT.insert(DzT.end(), DzzTd.begin(), DzzTd.end());
     p->xs = spectrum_xs(p->M, p->K);
     const size_t specN = (size_t)p->nx * p->xs, bcN = (size_t)2 * p->nx * p->M;
     if ((st = upload(&p->d_Dz, p->Dz)) || (st = upload(&p->d_Dzz, p->Dzz)) ||
-        (st = upload(&p->d_DzzT, DzzT)) || (st = dmalloc(&p->d_shift, p->modes)) ||
+        (st = upload(&p->d_DzzT, DzzT)) || (st = upload(&p->d_DzT, DzT)) || (st = derivative_prepare(p->N)) || (st = dmalloc(&p->d_shift, p->modes)) ||
         (st = upload(&p->d_twx, twiddles(p->nx))) || (st = upload(&p->d_twy, twiddles(p->ny))) ||
         (st = dmalloc(&p->spec.re, 2 * specN)) || (st = dmalloc(&p->bc.re, 2 * bcN)) ||
         (st = dmalloc(&p->d_status, p->modes)) ||

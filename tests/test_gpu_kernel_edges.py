@@ -1,0 +1,32 @@
+"""Kernel variants at the sizes where they can go wrong (tile edges,
+remainders, the smallest and largest of their range) against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+def to_dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("nx,ny,N,ne", [(1, 1, 3, 1), (2, 1, 16, 1), (1, 64, 17, 1), (8, 8, 32, 2), (4, 32, 33, 3),
+                                        (2, 64, 129, 1), (1, 128, 130, 1), (2, 32, 257, 1), (1, 16, 258, 1)])
+def test_derivative_z_tiles(cuda, nx, ny, N, ne):
+    """Whole and partial tiles of 64 columns, odd and even column strides,
+    one to 17 strips of 16 output rows, both orders: the products and sums of
+    the reference in its order, bit for bit."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    plan = HelmholtzPlan(nx, ny, N, ne, form="diag")
+    u = np.random.default_rng(N).standard_normal((ne, nx, ny, N))
+    du = to_dev(u)
+    for order, D in zip((1, 2), plan.operators()):
+        want = np.zeros_like(u)
+        for p in range(N):  # p ascending, every product rounded before it is added
+            want = want + D[:, p] * u[..., p:p + 1]
+        got = plan.derivative_z(du, order, out=torch.empty_like(du)).cpu().numpy()
+        assert np.array_equal(got, want), order
