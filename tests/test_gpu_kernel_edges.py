@@ -13,6 +13,33 @@ def to_dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
+def factored(n, count, seed, swaps=True):
+    """Reference factors and pivots of random systems (rows exchanged at
+    almost every step without `swaps` = False's dominant diagonal)."""
+    r = np.random.default_rng(seed)
+    A = r.standard_normal((count, n, n))
+    if not swaps:
+        A += 3 * n * np.eye(n)
+    b = r.standard_normal((count, n))
+    LU, piv, x = np.empty_like(A), np.zeros((count, max(n - 1, 1)), np.int32), np.empty_like(b)
+    for c in range(count):
+        lu, p, _ = po.lu(A[c])
+        LU[c], piv[c, :n - 1] = lu, p
+        x[c] = po.lu_solve(lu, p, b[c])
+    return LU, piv, b, x
+
+
+@pytest.mark.parametrize("n", [2, 3, 8, 9, 16, 17, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("swaps", [True, False])
+def test_lu_solve_every_size_class(cuda, n, swaps):
+    """One wave per system (one row per lane to 64, two to 128), and the
+    general kernel above: the reference's result bit for bit."""
+    from mpi_amd.solver import lu_solve_batched
+    LU, piv, b, x = factored(n, 5, n, swaps)
+    got = lu_solve_batched(to_dev(LU), to_dev(piv), to_dev(b)).cpu().numpy()
+    assert np.array_equal(got, x)
+
+
 @pytest.mark.parametrize("nx,ny,N,ne", [(1, 1, 3, 1), (2, 1, 16, 1), (1, 64, 17, 1), (8, 8, 32, 2), (4, 32, 33, 3),
                                         (2, 64, 129, 1), (1, 128, 130, 1), (2, 32, 257, 1), (1, 16, 258, 1)])
 def test_derivative_z_tiles(cuda, nx, ny, N, ne):
