@@ -57,3 +57,26 @@ def test_derivative_z_tiles(cuda, nx, ny, N, ne):
             want = want + D[:, p] * u[..., p:p + 1]
         got = plan.derivative_z(du, order, out=torch.empty_like(du)).cpu().numpy()
         assert np.array_equal(got, want), order
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65])
+@pytest.mark.parametrize("swaps", [True, False])
+def test_lu_factor_every_size_class(cuda, n, swaps):
+    """One wave per matrix (16, 32, 64 columns) and the work-group kernel
+    above: factors, pivots and determinant of the reference bit for bit, and a
+    singular matrix flagged."""
+    from mpi_amd.solver import lu_factor_batched
+    r = np.random.default_rng(n)
+    A = r.standard_normal((4, n, n)) + (0 if swaps else 3 * n * np.eye(n))
+    A[3] *= 1e-2 ** r.integers(0, 6, (n, 1))  # rows of very different scale
+    dA = to_dev(A)
+    piv, det, st = (t.cpu().numpy() for t in lu_factor_batched(dA))
+    LU = dA.cpu().numpy()
+    for c in range(4):
+        lu, p, d = po.lu(A[c])
+        assert np.array_equal(LU[c], lu) and list(piv[c, :n - 1]) == list(p[:n - 1]) and det[c] == d, c
+    assert not st.any()
+    if n > 1:
+        A[2, :, n // 2 if n > 2 else 0] = 0.0
+        st = lu_factor_batched(to_dev(A))[2].cpu().numpy()
+        assert list(st) == [0, 0, 4, 0]
