@@ -70,13 +70,14 @@ int launch_fft(int L, FftKind kind, const FftArgs &a, hipStream_t s);
 // Lane widths offered for length L (autotuned per plan); returns the count.
 int fft_width_choices(int L, int *w, int max);
 
-// Arguments of the plain-LU mode kernel (lu.hip).
+// Arguments of the plain-LU mode kernel (lu_modes.hip).
 struct LuModeArgs {
     int nx, ny, M, K, N, n, ne;
     long long xs;            // spectrum x-row stride (>= M * K)
     double *closure;         // periodic z: [re|im][nx * M] closure coefficients, or null
     const double *DzzT;      // interior operator transposed: DzzT[j*n + i] = Dzz[i+1][j+1]
     const double *Dzz;       // full N x N
+    const double *offmax;    // [n] max |Dzz[i+1][j+1]| over the interior j != i
     const double *Dz;        // full N x N
     const double *shift;     // [modes] or null
     const double *op_diag;   // [modes][n] or null
@@ -89,6 +90,9 @@ struct LuModeArgs {
     int cols;                // instance column capacity (lu_modes_shapes); 0 = the smallest
 };
 int launch_lu_modes(const LuModeArgs &a, int modes, hipStream_t s);
+int launch_lu_modes_above_64(const LuModeArgs &a, int modes, hipStream_t s);  // N - 2 > 64
+// The mode kernels' LDS limit on the current device (once per plan).
+int lu_modes_prepare();
 // Column capacities (16, 32, 64, 128) of the mode-kernel instances that hold
 // (nx, N-2, ne), smallest first; returns their number (at most `max` written).
 int lu_modes_shapes(int nx, int n, int ne, int *cols, int max);
@@ -229,7 +233,7 @@ struct hz_plan {
     double Lx = 0, Ly = 0, Lz = 0;
     std::vector<double> z, Dz, Dzz, shift;
     // device
-    double *d_Dz = nullptr, *d_Dzz = nullptr, *d_DzzT = nullptr, *d_shift = nullptr;
+    double *d_Dz = nullptr, *d_Dzz = nullptr, *d_DzzT = nullptr, *d_offmax = nullptr, *d_shift = nullptr;
     double *d_DzT = nullptr;  // hz_derivative_z's operands: Dz's, then (DzT_n further on) Dzz's
     size_t DzT_n = 0;
     double2 *d_twx = nullptr, *d_twy = nullptr;

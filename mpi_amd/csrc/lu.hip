@@ -1,5 +1,6 @@
-// lu.hip -- the reference algorithm per (|kx|,|ky|) mode: one work-group per
-// mode, the whole augmented system resident in registers.
+// lu.hip -- the reference algorithm per (|kx|,|ky|) mode for N - 2 above 64
+// (smaller operators: lu_modes.hip): one work-group per mode, the whole
+// augmented system resident in registers; and the standalone batched LU.
 //
 // For mode (iw, jw) the work-group
 //   1. assembles A = Dzz_int - sigma I (or the caller's operator) and the
@@ -35,6 +36,7 @@
 #include "hz_internal.h"
 #include "lu_slots.h"
 #include "sweep.h"
+#include "wave_ops.h"
 
 namespace hz {
 namespace {
@@ -48,14 +50,6 @@ constexpr int WAVE = 64;
 constexpr int kMaxRhs = 2 + 4 * 64;
 
 __host__ __device__ __forceinline__ int rhs_per_element(int nx) { return nx >= 4 ? 4 : 2; }
-
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // a - l*p with the product rounded before the difference
 // (LU_Decomposition.cpp:56-57 `A[l][m] -= A[l][k]*A[k][m]`).
@@ -330,58 +324,6 @@ __device__ __forceinline__ void eliminate(double (&A)[RB][CB], double (&Y)[RB][N
 }
 
 // ---- the mode kernel's elimination ------------------------------------------
-// Lane exchanges without LDS: DPP moves within rows of 16 lanes, readlane
-// across them.
-template <int CTRL>
-__device__ __forceinline__ int dpp_i32(int v)
-{
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
-}
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v)
-{
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)dpp_i32<CTRL>((int)(unsigned)b);
-    const unsigned hi = (unsigned)dpp_i32<CTRL>((int)(unsigned)(b >> 32));
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// v of lane l (l uniform)
-__device__ __forceinline__ double lane_f64(double v, int l)
-{
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// DPP controls: quad_perm [1,0,3,2] and [2,3,0,1] (lane xor 1, xor 2), then
-// the half-row and row mirrors, which leave every lane with the reduction
-// over its row of 16 lanes; the four rows are then combined by readlane.
-constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
-
-// Maximum of v over the wave (uniform result); v is not NaN.
-__device__ __forceinline__ double wave_max_f64(double v)
-{
-    v = fmax(v, dpp_f64<kDppXor1>(v));
-    v = fmax(v, dpp_f64<kDppXor2>(v));
-    v = fmax(v, dpp_f64<kDppHalfMirror>(v));
-    v = fmax(v, dpp_f64<kDppMirror>(v));
-    return fmax(fmax(lane_f64(v, 0), lane_f64(v, 16)), fmax(lane_f64(v, 32), lane_f64(v, 48)));
-}
-
-// Minimum of v over the wave (uniform result).
-__device__ __forceinline__ int wave_min_i32(int v)
-{
-    v = min(v, dpp_i32<kDppXor1>(v));
-    v = min(v, dpp_i32<kDppXor2>(v));
-    v = min(v, dpp_i32<kDppHalfMirror>(v));
-    v = min(v, dpp_i32<kDppMirror>(v));
-    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
-}
-
 // Pivot of position k (LU_Decomposition.cpp:32-49), run by the wave that
 // owns matrix column k with colv = that column brought up to date: the
 // candidate at position i >= k is |a_ik| / s_i (s: the original max-norm
@@ -1174,10 +1116,10 @@ __global__ void lu_solve_kernel(const double *LU, const int *piv, double *b, int
     }
 }
 
-template <int RB, int CB, int NR>
+template <int NR>
 int launch_modes_t(const LuModeArgs &a, int modes, hipStream_t s)
 {
-    hipLaunchKernelGGL((lu_modes_kernel<RB, CB, NR, 4>), dim3(modes), dim3(WAVE * 4), 0, s, a);
+    hipLaunchKernelGGL((lu_modes_kernel<2, 32, NR, 4>), dim3(modes), dim3(WAVE * 4), 0, s, a);
     HZ_HIP(hipGetLastError());
     return HZ_OK;
 }
@@ -1190,63 +1132,12 @@ int launch_factor_t(const LuFactorArgs &a, hipStream_t s)
     return HZ_OK;
 }
 
-template <int RB, int CB>
-int launch_modes_nr(const LuModeArgs &a, int modes, hipStream_t s)
-{
-    const int nr = (2 + rhs_per_element(a.nx) * a.ne + 3) / 4;  // right-hand sides per wave
-    if (nr <= 2) return launch_modes_t<RB, CB, 2>(a, modes, s);
-    if (nr <= 8) return launch_modes_t<RB, CB, 8>(a, modes, s);
-    if constexpr (RB == 1) {
-        if (nr <= 32) return launch_modes_t<1, CB, 32>(a, modes, s);
-        if (nr <= 64) return launch_modes_t<1, CB, 64>(a, modes, s);
-    }
-    return set_error(HZ_ERR_UNSUPPORTED, "PLAIN_LU form: too many elements (2 + c*ne right-hand sides, c = 4 "
-                                         "when nx >= 4 else 2, must be <= 256, or <= 32 when N-2 > 64)");
-}
-
 }  // namespace
 
-int lu_modes_check(int nx, int n, int ne)
+int launch_lu_modes_above_64(const LuModeArgs &a, int modes, hipStream_t s)
 {
-    if (n > 128) return set_error(HZ_ERR_UNSUPPORTED, "PLAIN_LU form: N-2 must be <= 128");
-    const int nrhs = 2 + rhs_per_element(nx) * ne;
-    if (nrhs > 4 * (n <= 64 ? 64 : 8))  // 4 waves x NR of the largest instance
-        return set_error(HZ_ERR_UNSUPPORTED, "PLAIN_LU form: too many elements (at most 63, or 127 when nx < 4; "
-                                             "7, or 15 when nx < 4, for N-2 > 64)");
-    return HZ_OK;
-}
-
-int lu_modes_shapes(int nx, int n, int ne, int *cols, int max)
-{
-    // column capacity 4*CB of the four instances: 64 rows (RB = 1) up to 64
-    // columns, then 128 rows and columns, whose right-hand sides stop at 8
-    // per wave; an instance holds every smaller n (masked columns, padding rows)
-    static const int caps[] = {16, 32, 64, 128};
-    const int nr = (2 + rhs_per_element(nx) * ne + 3) / 4;
-    int k = 0;
-    for (int cap : caps) {
-        if (cap < n || nr > (cap == 128 ? 8 : 64)) continue;
-        if (k < max) cols[k] = cap;
-        ++k;
-    }
-    return k;
-}
-
-int launch_lu_modes(const LuModeArgs &a, int modes, hipStream_t s)
-{
-    if (int st = lu_modes_check(a.nx, a.n, a.ne)) return st;
-    const int cols = a.cols ? a.cols : a.n <= 16 ? 16 : a.n <= 32 ? 32 : a.n <= 64 ? 64 : 128;
-    int c[4];
-    const int k = lu_modes_shapes(a.nx, a.n, a.ne, c, 4);
-    bool held = false;
-    for (int i = 0; i < k && i < 4; ++i) held = held || c[i] == cols;
-    if (!held) return set_error(HZ_ERR_ARG, "PLAIN_LU form: the mode-kernel shape does not hold this plan");
-    switch (cols) {
-    case 16: return launch_modes_nr<1, 4>(a, modes, s);
-    case 32: return launch_modes_nr<1, 8>(a, modes, s);
-    case 64: return launch_modes_nr<1, 16>(a, modes, s);
-    default: return launch_modes_nr<2, 32>(a, modes, s);
-    }
+    const int nr = (2 + rhs_per_element(a.nx) * a.ne + 3) / 4;  // right-hand sides per wave
+    return nr <= 2 ? launch_modes_t<2>(a, modes, s) : launch_modes_t<8>(a, modes, s);
 }
 
 int launch_lu_factor(const LuFactorArgs &a, hipStream_t s)

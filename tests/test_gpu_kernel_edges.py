@@ -80,3 +80,67 @@ def test_lu_factor_every_size_class(cuda, n, swaps):
         A[2, :, n // 2 if n > 2 else 0] = 0.0
         st = lu_factor_batched(to_dev(A))[2].cpu().numpy()
         assert list(st) == [0, 0, 4, 0]
+
+
+@pytest.mark.parametrize("N", [3, 9, 16, 17, 18, 19, 33, 34, 35, 50, 51, 65, 66])
+@pytest.mark.parametrize("scale", ["unit", "rows", "small", "huge"])
+def test_plain_panel_kernel_any_operator(cuda, N, scale):
+    """The mode kernel for N - 2 <= 64 (panels of 16 columns on 16 x 16
+    tiles) at its tile edges, on operators that exchange rows at almost every
+    step: rows of very different scale, pivots far from 1, and scales whose
+    reciprocals leave the ordinary range (the exact pivot comparison).  One
+    mode (1-D), Dirichlet ends: A u = f - Dzz[:,0] g_l - Dzz[:,-1] g_r."""
+    from mpi_amd.solver import HelmholtzPlan
+    n = N - 2
+    plan = HelmholtzPlan(1, 1, N, 1, form="plain")
+    r = np.random.default_rng(N)
+    A = r.standard_normal((n, n)) + (2.0 if n == 1 else 0.0)
+    s = {"unit": np.ones(n), "rows": 10.0 ** r.integers(-6, 7, n), "small": np.full(n, 2.0 ** -600),
+         "huge": np.full(n, 2.0 ** 1003)}[scale]
+    f = r.standard_normal(N)
+    b = f.copy()
+    b[1:-1] *= s
+    zero = to_dev(np.zeros((1, 1)))
+    u = plan.solve_operators(to_dev(b.reshape(1, 1, N)), zero, zero, op_full=to_dev((s[:, None] * A)[None]))
+    plan.status()
+    u = u.cpu().numpy().ravel()
+    want = np.linalg.solve(A, f[1:-1])
+    # backward stable elimination: n eps times the condition, and a growth of 8
+    tol = 8 * n * 2.0 ** -52 * np.linalg.cond(A) * np.abs(want).max()
+    assert u[0] == 0 and u[-1] == 0
+    assert np.abs(u[1:-1] - want).max() <= tol, (np.abs(u[1:-1] - want).max(), tol)
+    if n > 1:  # a zero column is singular
+        A[:, n // 2] = 0.0
+        plan.solve_operators(to_dev(b.reshape(1, 1, N)), zero, zero, op_full=to_dev((s[:, None] * A)[None]))
+        from mpi_amd._lib import HzError
+        with pytest.raises(HzError):
+            plan.status()
+    plan.close()
+
+
+@pytest.mark.parametrize("nx,ny,N,ne,periodic", [(1, 1, 8, 127, False), (4, 4, 10, 63, False), (4, 2, 66, 7, False),
+                                                 (2, 4, 66, 40, True), (4, 4, 18, 16, True), (4, 4, 34, 21, False)])
+def test_plain_panel_kernel_many_right_hand_sides(cuda, nx, ny, N, ne, periodic):
+    """Up to the largest number of right-hand sides (2 + c ne, c = 2 or 4), in
+    one and several groups of 64, against the diagonalised or the reference's
+    algorithm (the oracle), within twice the oracle's rounding spread."""
+    from mpi_amd.solver import HelmholtzPlan
+    lam = 3.0
+    plan = HelmholtzPlan(nx, ny, N, ne, xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2, lam=lam, form="plain",
+                         periodic_z=periodic)
+    r = np.random.default_rng(N + ne)
+    f = r.standard_normal((nx, ny, plan.nz))
+    if periodic:
+        f[:, :, -1] = f[:, :, 0]
+    g = [r.standard_normal((nx, ny)) for _ in range(2)]
+    desc = po.make_desc(nx, ny, ne * N, N, size=1, xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2, lam=lam)
+    if periodic:
+        uo, uf = po.solve_periodic(desc, f), po.solve_periodic(desc, f, fma=True)
+        u = plan.solve(to_dev(f))
+    else:
+        uo, uf = po.solve(desc, f, *g), po.solve(desc, f, *g, fma=True)
+        u = plan.solve(to_dev(f), *map(to_dev, g))
+    plan.status()
+    bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+    assert np.abs(u.cpu().numpy() - uo).max() / np.abs(uo).max() <= bar
+    plan.close()
