@@ -126,7 +126,8 @@ def whole_solve_roofline(form, ms_per_solve, nx, ny, n_gll, refine_sweeps=2, cei
 
 
 STAGE_KERNELS = {"diag_modes": "diag_modes_kernel", "lu_modes": "lu_modes_kernel",
-                 "fft_forward": "fft_lines", "fft_inverse": "fft_lines"}
+                 "fft_forward": "fft_lines", "fft_inverse": "fft_lines",
+                 "z_expand": "zf_expand", "xy_filter": "zf_filter", "z_collect": "zf_collect"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_256x256x129.json")
 
 
@@ -599,7 +600,8 @@ def main():
                         "tuner re-run right after the timed window, HIP events on its stream), stage_event_ms = "
                         "the stage's event pair inside a solve"}
     else:
-        work = fft_bytes(NX, NY, K) / 2
+        # a z-first stage reads and writes the interior once; the line passes of one direction
+        work = 2 * 8 * NX * NY * (K - 2) if stage in ("z_expand", "xy_filter", "z_collect") else fft_bytes(NX, NY, K) / 2
         roof = {"kernel": stage, "bound": "hbm", "achieved": work / (ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9,
                 "unit": "GB/s", "work_per_launch": work, "work_unit": "bytes"}
     roof["frac"] = roof["achieved"] / roof["peak"]

@@ -128,6 +128,31 @@ int diag_tile_choices(int NP, int *rt, int max);
 int launch_diag_modes(const DiagArgs &a, hipStream_t s);
 
 
+// The one-element Dirichlet solve with the z contractions outside the x-y
+// transforms (zfirst.hip), three launches: stage 0 expand, 1 filter, 2 collect.
+struct ZfArgs {
+    int nx, ny, K, n;
+    int lr2;                    // log2(ny / 16)
+    int ncol;                   // nx ny / 16 columns (x, n2)
+    const double *f;            // [nx][ny][K]: the right-hand side (adjoint: dL/du)
+    double *u;                  // [nx][ny][K]: the solution (adjoint: dL/df)
+    const double *gl, *gr;      // [nx][ny] (forward)
+    double *glbar, *grbar;      // [nx][ny] (adjoint)
+    double beta_l, beta_r;
+    double *T;                  // [n][8][ncol] complex
+    const double *B1, *B2;      // [NP][NP] contraction operands, row k, column j
+    const short *C1, *C2;       // correction, bf16 [NP/4][NP][4], and ..
+    const double *X1, *X2;      // .. its first 16 x 16 blocks in FP64 [2][k][j]
+    const double *w0, *wN;      // [NP] face loads in the eigenbasis
+    const double *mu;           // [n] eigenvalues, even ones first
+    const double *sx, *sy;      // shifts lambda + kx^2 [nx/2 + 1], ky^2 [ny/2 + 1]
+    const double2 *twx, *twy;
+    int adjoint, cubic;
+    double c3, c1;              // cubic: the right-hand side f (c3 f^2 + c1)
+};
+bool zf_holds(int nx, int ny, int n);
+int launch_zf(const ZfArgs &a, int stage, hipStream_t s);
+
 // MIXED form (mixed.hip, mixed_body.h): FP32 eigenbasis solves refined with
 // FP64 residuals, both on the matrix cores.
 struct MixedSetupArgs {
@@ -254,6 +279,12 @@ struct hz_plan {
     double *d_eo_vec = nullptr, *d_eo_B1 = nullptr, *d_eo_B2 = nullptr, *d_eo_hom = nullptr;
     double *d_eo_B1a = nullptr, *d_eo_B2a = nullptr;  // adjoint operands
     short *d_eo_M = nullptr, *d_eo_Ma = nullptr;      // first-order correction (bf16), forward and adjoint
+    // z-first solve (zfirst.hip), where it applies: the operands in one
+    // allocation (forward B1, B2, X1, X2, then the adjoint's; w0, wN, mu), the
+    // bf16 corrections in another, and the shifts' two parts
+    bool zf = false;
+    double *d_zf = nullptr, *d_zf_shift = nullptr;
+    short *d_zf_C = nullptr;
     int diag_rt = 0;                                  // autotuned tile rows
     int lu_cols = 0;                                  // autotuned PLAIN instance (0 = smallest)
     std::vector<double> lu_cols_ms;                   // tuning times per LU instance

@@ -82,6 +82,9 @@ void free_plan(hz_plan *p)
                       p->d_Vinvrow, p->d_eo_vec, p->d_eo_B1, p->d_eo_B2, p->d_eo_B1a, p->d_eo_B2a, p->d_eo_hom,
                       p->d_partial, p->d_DzzTP, p->d_UL, p->d_UR, p->d_hist, p->d_closure})
         (void)hipFree(q);
+    (void)hipFree(p->d_zf);
+    (void)hipFree(p->d_zf_shift);
+    (void)hipFree(p->d_zf_C);
     (void)hipFree(p->d_eo_M);
     (void)hipFree(p->d_eo_Ma);
     (void)hipFree(p->d_VinvT32);
@@ -184,6 +187,18 @@ int setup_mixed(hz_plan *p)
     return HZ_OK;
 }
 
+// The shift's two parts of the z-first solve, lambda + kx^2 and ky^2: their
+// sum is mode_shift's, bit for bit.
+int zf_shifts(hz_plan *p)
+{
+    if (!p->zf) return HZ_OK;
+    std::vector<double> v;
+    for (int iw = 0; iw <= p->nx / 2; ++iw) v.push_back(mode_shift(p->d.lambda, iw, 0, p->Lx, p->Ly));
+    for (int jw = 0; jw < p->M; ++jw) v.push_back(mode_shift(0.0, 0, jw, p->Lx, p->Ly));
+    HZ_HIP(hipMemcpy(p->d_zf_shift, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice));
+    return HZ_OK;
+}
+
 int compute_shifts(hz_plan *p)
 {
     p->shift.resize(p->modes);
@@ -193,6 +208,7 @@ int compute_shifts(hz_plan *p)
     HZ_HIP(hipMemcpy(p->d_shift, p->shift.data(), sizeof(double) * p->modes, hipMemcpyHostToDevice));
     int st = compute_homogeneous(p);
     if (st) return st;
+    if ((st = zf_shifts(p))) return st;
     if (p->d.form == HZ_FORM_MIXED && p->d_UL) return mixed_operators(p);
     return HZ_OK;
 }
@@ -212,10 +228,20 @@ int compute_shifts(hz_plan *p)
 // differences of mirrored entries (the halves of F^-1 are folded into D W,
 // D = 1/2 except on the centre row of an odd n).  Operands, NP x NP
 // row-major: B1 = Winv^T, B2 = (D W)^T, adjoint B1 = D W, B2 = Winv (FP64),
-// M and M^T in bf16 (correction_operator); r0|rN =
+// M and M^T in bf16 (correction_operator); plans that the z-first solve holds
+// get its operands too (zf_operands); r0|rN =
 // Dz[0|N-1][1..N-2] F^-1 W (the homogeneous coefficients' basis).
-std::array<std::vector<short>, 2> correction_operator(const std::vector<double> &A, int n, int NP,
-                                                      const std::vector<double> &W, const std::vector<double> &Wi);
+std::vector<long double> correction_matrix(const std::vector<double> &A, int n, int NP, const std::vector<double> &W,
+                                           const std::vector<double> &Wi);
+std::array<std::vector<short>, 2> correction_operator(const std::vector<long double> &M, int NP);
+// zfirst.hip's operands of a plan (zf_operands): the FP64 ones, the bf16 ones.
+struct ZfOperands {
+    std::vector<double> d;
+    std::vector<short> c;
+};
+ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::vector<double> &W,
+                       const std::vector<double> &Wi, const std::vector<long double> &M,
+                       const std::vector<long double> &fg0, const std::vector<long double> &fgN);
 
 int setup_even_odd(hz_plan *p, const std::vector<double> &A)
 {
@@ -223,6 +249,10 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
     static std::mutex cache_mu;
     static std::map<std::pair<std::vector<double>, int>, std::array<std::vector<double>, 3>> cache;
     static std::map<std::pair<std::vector<double>, int>, std::array<std::vector<short>, 2>> cache_m;
+    static std::map<std::pair<std::vector<double>, int>, ZfOperands> cache_zf;
+    // one element, Dirichlet faces, and a grid that the z-first kernels hold
+    const bool zf = zf_holds(p->nx, p->ny, n) && !diag_general(p);
+    ZfOperands zo;
     std::vector<double> mu, W, Wi;
     std::array<std::vector<short>, 2> Mq;
     const auto key = std::make_pair(A, NP);
@@ -234,6 +264,10 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
             W = it->second[1];
             Wi = it->second[2];
             Mq = cache_m[key];
+            if (zf) {
+                auto z = cache_zf.find(key);
+                if (z != cache_zf.end()) zo = z->second;
+            }
         } else {
             const int st = eigen_decompose_split(A, n, NP, mu, W, Wi, nullptr);
             if (st) return set_error(st, "even/odd eigendecomposition of the GLL operator failed");
@@ -295,12 +329,15 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
             B2a[(size_t)r * NP + c] = Wi[(size_t)r * NP + c];
         }
     }
-    if (Mq[0].empty()) {
-        Mq = correction_operator(A, n, NP, W, Wi);
+    if (Mq[0].empty() || (zf && zo.d.empty())) {
+        const std::vector<long double> M = correction_matrix(A, n, NP, W, Wi);
+        Mq = correction_operator(M, NP);
+        if (zf) zo = zf_operands(n, NP, mu, W, Wi, M, fg0, fgN);
         std::lock_guard<std::mutex> lk(cache_mu);
-        if (cache.size() < 256) {
+        if (cache.size() < 256 || cache.count(key)) {
             cache[key] = {mu, W, Wi};
             cache_m[key] = Mq;
+            if (zf) cache_zf[key] = zo;
         }
     }
     int st;
@@ -308,21 +345,24 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
         (st = upload(&p->d_eo_B1a, B1a)) || (st = upload(&p->d_eo_B2a, B2a)) || (st = upload(&p->d_eo_M, Mq[0])) ||
         (st = upload(&p->d_eo_Ma, Mq[1])))
         return st;
+    if (zf) {
+        if ((st = upload(&p->d_zf, zo.d)) || (st = upload(&p->d_zf_C, zo.c)) ||
+            (st = dmalloc(&p->d_zf_shift, (size_t)p->nx / 2 + 1 + p->M)))
+            return st;
+        p->zf = true;
+    }
     return HZ_OK;
 }
 
 // The even/odd solve's first-order correction M = Winv (F Ea F^-1) W, Ea =
 // (A - JAJ)/2 (the middle factor column by column: F^-1 of a unit vector has
-// one or two entries; then the two products, in long double), as the bf16
-// B operands of c = M z (forward) and c = M^T q (adjoint):
-// [0][(k / 4) * NP + j][k % 4] = bf16(M[j][k]), [1][...] = bf16(M[k][j]),
-// rounded to nearest even.
-std::array<std::vector<short>, 2> correction_operator(const std::vector<double> &A, int n, int NP,
-                                                      const std::vector<double> &W, const std::vector<double> &Wi)
+// one or two entries; then the two products, in long double), NP x NP.
+std::vector<long double> correction_matrix(const std::vector<double> &A, int n, int NP, const std::vector<double> &W,
+                                           const std::vector<double> &Wi)
 {
     const int H = NP / 2, m = n / 2;
     typedef long double ld;
-    std::vector<ld> Et((size_t)NP * NP, 0), T((size_t)NP * NP, 0);
+    std::vector<ld> Et((size_t)NP * NP, 0), T((size_t)NP * NP, 0), M((size_t)NP * NP, 0);
     std::vector<ld> y(n);
     auto ea = [&](int r, int c) {
         return ((ld)A[(size_t)r * n + c] - (ld)A[(size_t)(n - 1 - r) * n + (n - 1 - c)]) / 2;
@@ -345,21 +385,126 @@ std::array<std::vector<short>, 2> correction_operator(const std::vector<double> 
             if (e == 0) continue;
             for (int c = 0; c < NP; ++c) T[(size_t)r * NP + c] += e * (ld)W[(size_t)k * NP + c];
         }
+    for (int r = 0; r < NP; ++r)      // M = Winv T
+        for (int k = 0; k < NP; ++k) {
+            const ld w = Wi[(size_t)r * NP + k];
+            if (w == 0) continue;
+            for (int c = 0; c < NP; ++c) M[(size_t)r * NP + c] += w * T[(size_t)k * NP + c];
+        }
+    return M;
+}
+
+// x rounded to bf16 (nearest even, through FP32), its upper 16 bits.
+short bf16_of(double x)
+{
+    const float f = (float)x;
+    uint32_t u;
+    std::memcpy(&u, &f, 4);
+    u += 0x7FFFu + ((u >> 16) & 1u);
+    return (short)(u >> 16);
+}
+
+double bf16_value(short b)
+{
+    const uint32_t u = (uint32_t)(uint16_t)b << 16;
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+}
+
+// M as the bf16 B operands of c = M z (forward) and c = M^T q (adjoint):
+// [0][(k / 4) * NP + j][k % 4] = bf16(M[j][k]), [1][...] = bf16(M[k][j]).
+std::array<std::vector<short>, 2> correction_operator(const std::vector<long double> &M, int NP)
+{
     std::array<std::vector<short>, 2> Mq;
     Mq[0].assign((size_t)NP * NP, 0);
     Mq[1].assign((size_t)NP * NP, 0);
-    for (int r = 0; r < NP; ++r)      // M = Winv T
+    for (int r = 0; r < NP; ++r)
         for (int c = 0; c < NP; ++c) {
-            ld acc = 0;
-            for (int k = 0; k < NP; ++k) acc += (ld)Wi[(size_t)r * NP + k] * T[(size_t)k * NP + c];
-            const float f = (float)acc;
-            uint32_t u;
-            std::memcpy(&u, &f, 4);
-            u += 0x7FFFu + ((u >> 16) & 1u);
-            Mq[0][((size_t)(c / 4) * NP + r) * 4 + c % 4] = (short)(u >> 16);  // B[k = c][j = r]
-            Mq[1][((size_t)(r / 4) * NP + c) * 4 + r % 4] = (short)(u >> 16);  // B[k = r][j = c]
+            const short b = bf16_of((double)M[(size_t)r * NP + c]);
+            Mq[0][((size_t)(c / 4) * NP + r) * 4 + c % 4] = b;  // B[k = c][j = r]
+            Mq[1][((size_t)(r / 4) * NP + c) * 4 + r % 4] = b;  // B[k = r][j = c]
         }
     return Mq;
+}
+
+// The z-first solve's operands (zfirst.hip) from the even/odd decomposition
+// and M: G_ij = M_ij / (mu_j - mu_i) between the halves, its entries outside
+// the first 16 x 16 block of each half rounded to bf16 as the kernels use
+// them, K = (I - G^2)^-1 (= I + G^2 + G^4 here: G^2 <= 1e-8).  With KW = K
+// Winv: forward B1 = KW^T, -G; B2 = (D W)^T, +G; adjoint B1 = D W, +G^T; B2 =
+// KW, -G^T; face loads K Winv F g: added before the correction (forward), or
+// against the corrected z (adjoint).  `d`: [B1, B2, X1, X2, w0, wN] forward, then
+// adjoint, then the n eigenvalues, even ones first; `c`: the four bf16 parts.
+ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::vector<double> &W,
+                       const std::vector<double> &Wi, const std::vector<long double> &M,
+                       const std::vector<long double> &fg0, const std::vector<long double> &fgN)
+{
+    const int H = NP / 2, ho = n / 2, he = n - ho;
+    const size_t Q = (size_t)NP * NP;
+    auto real = [&](int j) { return j < H ? j < he : j - H < ho; };
+    auto at = [&](std::vector<double> &v, int i, int j) -> double & { return v[(size_t)i * NP + j]; };
+    std::vector<double> G(Q, 0.0), G2(Q, 0.0), KW(Q, 0.0), K(Q, 0.0);
+    ZfOperands o;
+    const size_t set = 2 * Q + 1024 + 2 * NP;
+    o.d.assign(2 * set + n, 0.0);
+    o.c.assign(4 * Q, 0);
+    for (int i = 0; i < NP; ++i)
+        for (int j = 0; j < NP; ++j) {
+            if (!real(i) || !real(j) || (i < H) == (j < H)) continue;
+            const double g = (double)(M[(size_t)i * NP + j] / ((long double)mu[j] - (long double)mu[i]));
+            const bool block = i % H < 16 && j % H < 16;
+            at(G, i, j) = block ? g : bf16_value(bf16_of(g));
+        }
+    auto product = [&](std::vector<double> &out, const std::vector<double> &a, const std::vector<double> &b) {
+        for (int i = 0; i < NP; ++i)
+            for (int k = 0; k < NP; ++k) {
+                const double v = a[(size_t)i * NP + k];
+                if (v == 0) continue;
+                for (int j = 0; j < NP; ++j) out[(size_t)i * NP + j] += v * b[(size_t)k * NP + j];
+            }
+    };
+    product(G2, G, G);
+    K = G2;
+    product(K, G2, G2);
+    KW = Wi;
+    product(KW, K, Wi);  // (I + G^2 + G^4) Winv
+    double *f = o.d.data(), *ad = o.d.data() + set;
+    for (int k = 0; k < NP; ++k)
+        for (int j = 0; j < NP; ++j) {
+            auto dw = [&](int r, int c) { return (n % 2 && r == n / 2 ? 1.0 : 0.5) * W[(size_t)r * NP + c]; };
+            f[(size_t)k * NP + j] = at(KW, j, k);
+            f[Q + (size_t)k * NP + j] = dw(j, k);
+            ad[(size_t)k * NP + j] = dw(k, j);
+            ad[Q + (size_t)k * NP + j] = at(KW, k, j);
+            if ((k < H) == (j < H)) continue;
+            const double g = at(G, j, k), gt = at(G, k, j);
+            if (k % H < 16 && j % H < 16) {
+                const size_t x = 2 * Q + (j < H ? 0 : 256) + (size_t)(k % H) * 16 + j % H;
+                f[x] = -g;
+                f[x + 512] = g;
+                ad[x] = gt;
+                ad[x + 512] = -gt;
+            } else {
+                const size_t x = ((size_t)(k / 4) * NP + j) * 4 + k % 4;
+                o.c[x] = bf16_of(-g);
+                o.c[Q + x] = bf16_of(g);
+                o.c[2 * Q + x] = bf16_of(gt);
+                o.c[3 * Q + x] = bf16_of(-gt);
+            }
+        }
+    const size_t vec = 2 * Q + 1024;
+    for (int side = 0; side < 2; ++side) {
+        const std::vector<long double> &fg = side ? fgN : fg0;
+        std::vector<long double> w(NP, 0);
+        for (int j = 0; j < NP; ++j)
+            for (int k = 0; k < NP; ++k) w[j] += (long double)at(KW, j, k) * fg[k];
+        for (int j = 0; j < NP; ++j)
+            f[vec + (size_t)side * NP + j] = ad[vec + (size_t)side * NP + j] = real(j) ? (double)w[j] : 0.0;
+    }
+    for (int j = 0; j < he; ++j) o.d[2 * set + j] = mu[j];
+    for (int j = 0; j < ho; ++j) o.d[2 * set + he + j] = mu[H + j];
+    return o;
 }
 
 // Eigen-decomposition of the interior operator and the derived vectors of
@@ -1036,6 +1181,59 @@ int hz_plan_set_robin(hz_plan *p, double alpha_l, double beta_l, double alpha_r,
     return HZ_OK;
 }
 
+// The one-element Dirichlet solve or its adjoint (f = dL/du, u = dL/df) with
+// the z contractions outside the transforms (zfirst.hip); the plan's spectrum
+// is the intermediate.
+static int zf_pipeline(hz_plan *p, const double *f, double *u, const double *gl, const double *gr, double *glbar,
+                       double *grbar, const double *cubic, hipStream_t s, StageRecorder *rec)
+{
+    const size_t Q = (size_t)p->NP * p->NP, set = 2 * Q + 1024 + 2 * p->NP;
+    const bool adj = glbar != nullptr;
+    const double *d = p->d_zf + (adj ? set : 0);
+    const short *c = p->d_zf_C + (adj ? 2 * Q : 0);
+    ZfArgs a{};
+    a.nx = p->nx;
+    a.ny = p->ny;
+    a.K = p->K;
+    a.n = p->n;
+    while ((16 << a.lr2) < p->ny) ++a.lr2;
+    a.ncol = p->nx << a.lr2;
+    a.f = f;
+    a.u = u;
+    a.gl = gl;
+    a.gr = gr;
+    a.glbar = glbar;
+    a.grbar = grbar;
+    a.beta_l = p->d.beta_l;
+    a.beta_r = p->d.beta_r;
+    a.T = p->spec.re;
+    a.B1 = d;
+    a.B2 = d + Q;
+    a.X1 = d + 2 * Q;
+    a.X2 = a.X1 + 512;
+    a.w0 = a.X2 + 512;
+    a.wN = a.w0 + p->NP;
+    a.C1 = c;
+    a.C2 = c + Q;
+    a.mu = p->d_zf + 2 * set;
+    a.sx = p->d_zf_shift;
+    a.sy = p->d_zf_shift + p->nx / 2 + 1;
+    a.twx = p->d_twx;
+    a.twy = p->d_twy;
+    a.adjoint = adj;
+    if (cubic) {
+        a.cubic = 1;
+        a.c3 = cubic[0];
+        a.c1 = cubic[1];
+    }
+    static const char *const names[3] = {"z_expand", "xy_filter", "z_collect"};
+    for (int stage = 0; stage < 3; ++stage) {
+        if (int st = launch_zf(a, stage, s)) return st;
+        if (rec) rec->mark(names[stage]);
+    }
+    return HZ_OK;
+}
+
 static int solve_impl(hz_plan *p, const double *f, const double *gl, const double *gr,
                       const double *op_diag, const double *op_full, double *u, hipStream_t s,
                       const double *cubic = nullptr)
@@ -1047,6 +1245,8 @@ static int solve_impl(hz_plan *p, const double *f, const double *gl, const doubl
         return set_error(HZ_ERR_ARG, "null face data");
     }
     StageRecorder rec(p, s);
+    if (p->d.form == HZ_FORM_DIAG && p->zf && !diag_general(p) && !op_diag && !op_full)
+        return zf_pipeline(p, f, u, gl, gr, nullptr, nullptr, cubic, s, &rec);
     int st = forward_xy(p, f, p->spec.re, p->spec.im, p->K, s, gl, gr, p->xs, cubic);
     rec.mark("fft_forward");
     if (st) return st;
@@ -1160,6 +1360,7 @@ static int adjoint_pipeline(hz_plan *p, const double *ubar, double *fbar, double
                             hipStream_t s, StageRecorder *rec)
 {
     int st;
+    if (p->zf && !diag_general(p)) return zf_pipeline(p, ubar, fbar, nullptr, nullptr, glbar, grbar, nullptr, s, rec);
     if ((st = forward_xy(p, ubar, p->spec.re, p->spec.im, p->K, s, nullptr, nullptr, p->xs))) return st;
     if (rec) rec->mark("fft_forward");
     DiagArgs a = diag_args(p);
@@ -1210,7 +1411,7 @@ int hz_adjoint(hz_plan *p, const double *ubar, const double *u, double *fbar, do
     if ((st = adjoint_args(p, ubar, u, fbar, glbar, grbar, lambda_bar))) return st;
     const hipStream_t s = (hipStream_t)stream;
     if (!p->d_Vrow) {
-        if ((st = setup_diag(p)) || (st = compute_homogeneous(p))) return st;
+        if ((st = setup_diag(p)) || (st = compute_homogeneous(p)) || (st = zf_shifts(p))) return st;
     }
     StageRecorder rec(p, s);
     if ((st = adjoint_pipeline(p, ubar, fbar, glbar, grbar, s, &rec))) return st;

@@ -144,3 +144,46 @@ def test_plain_panel_kernel_many_right_hand_sides(cuda, nx, ny, N, ne, periodic)
     bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
     assert np.abs(u.cpu().numpy() - uo).max() / np.abs(uo).max() <= bar
     plan.close()
+
+
+@pytest.mark.parametrize("nx,ny,N", [(64, 128, 66), (128, 64, 67), (256, 32, 98), (64, 256, 3), (128, 128, 4),
+                                     (256, 64, 17), (64, 256, 18), (128, 256, 19), (256, 128, 34), (256, 256, 5),
+                                     (128, 128, 35), (256, 64, 66), (64, 128, 99), (128, 64, 129), (256, 32, 130)])
+def test_z_first_solve_every_grid(cuda, nx, ny, N):
+    """The one-element Dirichlet DIAG solve with the z contractions outside
+    the transforms: every grid it holds, N - 2 at the edges of the matrix
+    tiles, end values scaled by beta.  Solve against the oracle within twice
+    its rounding spread (or 1e-12); right-hand side a3 u^3 + a1 u bit for bit
+    the solve of that field; adjoint (and solve) against the general path,
+    which a vanishing Robin term selects, each side within that bar."""
+    import torch
+    from mpi_amd import _lib
+    from mpi_amd.solver import HelmholtzPlan
+    lam, bl, br = 3.0, 2.0, -0.5
+    geo = dict(xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2)
+    plan = HelmholtzPlan(nx, ny, N, 1, lam=1.0, beta_l=bl, beta_r=br, form="diag", **geo)
+    plan.set_lambda(lam)
+    r = np.random.default_rng(nx + ny + N)
+    f = r.standard_normal((nx, ny, N))
+    g = [r.standard_normal((nx, ny)) for _ in range(2)]
+    df, dg = to_dev(f), [to_dev(v) for v in g]
+    desc = po.make_desc(nx, ny, N, N, size=1, lam=lam, betal=bl, betar=br, **geo)
+    uo, uf = po.solve(desc, f, *g), po.solve(desc, f, *g, fma=True)
+    bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+    plan.profile(True)
+    u = plan.solve(df, *dg)
+    assert "xy_filter" in plan.profile_read()[0]
+    plan.profile(False)
+    assert np.abs(u.cpu().numpy() - uo).max() <= bar * np.abs(uo).max()
+    lib = _lib.load()
+    cub = torch.empty_like(df)
+    _lib.check(lib.hz_cubic_rhs(df.data_ptr(), cub.data_ptr(), df.numel(), 0.5, -2.0,
+                                torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(plan.solve_cubic(df, 0.5, -2.0, *dg), plan.solve(cub, *dg))
+    other = HelmholtzPlan(nx, ny, N, 1, lam=lam, alpha_l=1e-300, beta_l=bl, alpha_r=1e-300, beta_r=br, form="diag",
+                          **geo)
+    pairs = [(u, other.solve(df, *dg))] + list(zip(plan.adjoint(df)[:3], other.adjoint(df)[:3]))
+    for got, want in pairs:
+        assert float((got - want).abs().max()) <= 2 * bar * float(want.abs().max())
+    plan.close()
+    other.close()
