@@ -201,6 +201,12 @@ int launch_derivative(const double *DT, int N, long long ncols, const double *u,
 // axis A (axis_a) or B of length L (Fourier derivative).
 int launch_spectral_derivative(double *re, double *im, long long A, long long B, long long lanes, int axis_a, int L,
                                double len, int order, hipStream_t s);
+// The same derivative in one pass over the field (fderiv.hip): nbatch batches
+// (stride bs) of `lanes` contiguous lines of L points at stride ps; tw is L's
+// twiddle table.  In place or on disjoint buffers.
+bool derivative_lines_holds(int L, long long nbatch, long long lanes);
+int launch_derivative_lines(int L, long long nbatch, long long lanes, long long bs, long long ps, const double *u,
+                            double *out, double len, int order, const double2 *tw, hipStream_t s);
 // sum_i a[i]*b[i] into *out (device or pinned host memory), deterministic two-pass reduction;
 // partial >= kDotPartials doubles (the first pass runs at most that many work-groups)
 constexpr int kDotPartials = 1024;

@@ -1531,9 +1531,10 @@ int hz_mixed_fp64_modes(const hz_plan *p, int *fp64_modes)
     return HZ_OK;
 }
 
-// Fourier derivative along x or y: one R2C pass along that axis into a half
-// spectrum, the wavenumber multiply, one C2R pass back (two passes over the
-// field, not the four of the 2-D transform).
+// Fourier derivative along x or y.  Lines of 32 to 256 points: one pass
+// (fderiv.hip).  Other lengths, and an output that overlaps the input without
+// being it: one R2C pass along that axis into a half spectrum, the wavenumber
+// multiply, one C2R pass back.
 int hz_derivative_xy(hz_plan *p, int axis, int order, const double *u, double *out, int lanes,
                      hz_stream_t stream)
 {
@@ -1541,6 +1542,16 @@ int hz_derivative_xy(hz_plan *p, int axis, int order, const double *u, double *o
         return set_error(HZ_ERR_ARG, "bad argument");
     const hipStream_t s = (hipStream_t)stream;
     const long long W = lanes;
+    {
+        const long long total = (long long)p->nx * p->ny * W;
+        const bool apart = u == out || out + total <= u || u + total <= out;
+        // along x the lanes of every y follow each other: one batch of ny W lanes
+        const long long nb = axis == 0 ? 1 : p->nx, ln = axis == 0 ? p->ny * W : W;
+        const int len = axis == 0 ? p->nx : p->ny;
+        if (apart && derivative_lines_holds(len, nb, ln))
+            return launch_derivative_lines(len, nb, ln, p->ny * W, ln, u, out, axis == 0 ? p->Lx : p->Ly, order,
+                                           axis == 0 ? p->d_twx : p->d_twy, s);
+    }
     const long long A = axis == 0 ? p->nx / 2 + 1 : p->nx;
     const long long B = axis == 0 ? p->ny : p->M;
     const size_t half = (size_t)A * B * W;
