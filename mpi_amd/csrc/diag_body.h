@@ -53,14 +53,13 @@
 
 #include "hz_internal.h"
 #include "sweep.h"
+#include "wave_ops.h"
 
 namespace hz {
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 constexpr int WAVE = 64;
-
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // acc[rb][jt] += A B over the k index, A = the LDS tile (rows
 // 16 (r0 + rb) + i, column k), B[k][j] = B[k * NP + j] from L2 (j in the

@@ -219,3 +219,34 @@ def test_fourier_derivative_lines(cuda, nx, ny, lanes, order):
         plan.derivative_xy(src, axis, order, out=dst)
         assert np.abs(dst.cpu().numpy() - want).max() <= tol
     plan.close()
+
+
+@pytest.mark.parametrize("N", [3, 4, 17, 18, 19, 34, 35, 66, 67, 98, 99, 130])
+@pytest.mark.parametrize("faces,ne", [("dirichlet", 1), ("robin", 1), ("robin", 3), ("periodic", 1), ("periodic", 8)])
+def test_mixed_one_wave_per_16_columns(cuda, N, faces, ne):
+    """The MIXED mode solve for N - 2 <= 128 at the edges of its column tiles,
+    with whole and partial row tiles, against the oracle within twice its
+    rounding spread (or 1e-12), and its residual history present and falling."""
+    from mpi_amd.solver import HelmholtzPlan
+    nx, ny, lam = 4, 8, 3.0
+    ab = (0.7, 1.3, 0.4, 2.0) if faces == "robin" else (0.0, 2.0, 0.0, -0.5)
+    geo = dict(xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2)
+    kw = {} if faces == "periodic" else dict(alpha_l=ab[0], beta_l=ab[1], alpha_r=ab[2], beta_r=ab[3])
+    plan = HelmholtzPlan(nx, ny, N, ne, lam=lam, form="mixed", periodic_z=faces == "periodic", **geo, **kw)
+    r = np.random.default_rng(N + ne)
+    f = r.standard_normal((nx, ny, plan.nz))
+    g = [r.standard_normal((nx, ny)) for _ in range(2)]
+    dk = {} if faces == "periodic" else dict(alphal=ab[0], betal=ab[1], alphar=ab[2], betar=ab[3])
+    desc = po.make_desc(nx, ny, ne * N, N, size=1, lam=lam, **geo, **dk)
+    if faces == "periodic":
+        f[:, :, -1] = f[:, :, 0]
+        uo, uf = po.solve_periodic(desc, f), po.solve_periodic(desc, f, fma=True)
+        u = plan.solve(to_dev(f))
+    else:
+        uo, uf = po.solve(desc, f, *g), po.solve(desc, f, *g, fma=True)
+        u = plan.solve(to_dev(f), *map(to_dev, g))
+    bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+    assert np.abs(u.cpu().numpy() - uo).max() <= bar * np.abs(uo).max()
+    h = plan.mixed_history()
+    assert len(h) == 2 and 0 < h[1] < h[0] < 1e-3
+    plan.close()
