@@ -95,9 +95,10 @@ __device__ __forceinline__ void dft_regs(double (&re)[R], double (&im)[R], const
 // Addressing of a tile's operands.  Point p of the thread's line is at
 // element index off(p) = base_offset + p * point_stride of each operand.
 // Addr64T: per-thread pointers and 64-bit indices (any lane mix, any size).
-// A lane with `cub` set reads x * (c3 x^2 + c1) for the real input x (the
+// A lane with `cub` set takes x * (c3 x^2 + c1) for the real input x (the
 // cubic right-hand side hz_solve_cubic forms inside the R2C pass; the same
-// operations as hz_cubic_rhs).  Only the CUB instances of the tile functions
+// operations as hz_cubic_rhs).  map() follows once every load is in flight:
+// formed point by point at the loads, each waited for its own.  Only the CUB instances of the tile functions
 // carry the map, so the plain transforms keep their loads as they are.
 __device__ __forceinline__ double cubic_map(double x, bool cub, double c3, double c1)
 {
@@ -113,10 +114,9 @@ struct Addr64T {
     double c3, c1;
     __device__ __forceinline__ double ldr(int p) const
     {
-        const double v = ire[ib + (long long)p * ips];
-        if constexpr (CUB) return cubic_map(v, cub, c3, c1);
-        return v;
+        return ire[ib + (long long)p * ips];
     }
+    __device__ __forceinline__ double map(double v) const { return CUB ? cubic_map(v, cub, c3, c1) : v; }
     __device__ __forceinline__ double ldi(int p) const { return iim[ib + (long long)p * ips]; }
     __device__ __forceinline__ void str(int p, double v) const { ore[ob + (long long)p * ops] = v; }
     __device__ __forceinline__ void sti(int p, double v) const { oim[ob + (long long)p * ops] = v; }
@@ -139,10 +139,9 @@ struct Addr32T {
     }
     __device__ __forceinline__ double ldr(int p) const
     {
-        const double v = *at(ire, ib + (unsigned)p * ips);
-        if constexpr (CUB) return cubic_map(v, cub, c3, c1);
-        return v;
+        return *at(ire, ib + (unsigned)p * ips);
     }
+    __device__ __forceinline__ double map(double v) const { return CUB ? cubic_map(v, cub, c3, c1) : v; }
     __device__ __forceinline__ double ldi(int p) const { return *at(iim, ib + (unsigned)p * ips); }
     __device__ __forceinline__ void str(int p, double v) const { *at(ore, ob + (unsigned)p * ops) = v; }
     __device__ __forceinline__ void sti(int p, double v) const { *at(oim, ob + (unsigned)p * ops) = v; }
@@ -191,6 +190,10 @@ __device__ __forceinline__ void fft_core(const A &ad, bool live, const double2 *
             }
             sre[n1] = vr;
             sim[n1] = vi;
+        }
+        if constexpr (KIND == FFT_R2C) {
+#pragma unroll
+            for (int n1 = 0; n1 < R1; ++n1) sre[n1] = ad.map(sre[n1]);
         }
     }
     if (q < R2) {
@@ -375,6 +378,10 @@ __device__ __forceinline__ void fft_core3(const A &ad, bool live, const double2 
             }
             sre[n1] = vr;
             sim[n1] = vi;
+        }
+        if constexpr (KIND == FFT_R2C) {
+#pragma unroll
+            for (int n1 = 0; n1 < R1; ++n1) sre[n1] = ad.map(sre[n1]);
         }
     }
     if (q < M) {
