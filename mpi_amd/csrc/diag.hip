@@ -22,14 +22,16 @@ int launch_t(const DiagArgs &a, hipStream_t s)
     const int blocks = (nfc + fc_per_tile - 1) / fc_per_tile;
     const bool general = a.ne > 1 || a.alpha_l != 0.0 || a.alpha_r != 0.0 || a.periodic;
     if (a.eo == general) return set_error(HZ_ERR_ARG, "DIAG form: the even/odd basis is for one Dirichlet element");
-    if (a.adjoint && a.eo) {
-        hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, false, true, true>), dim3(blocks), dim3(256), 0, s, a);
-    } else if (a.adjoint) {
-        hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, false, true, false>), dim3(blocks), dim3(256), 0, s, a);
-    } else if (general) {
-        hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, true, false, false>), dim3(blocks), dim3(256), 0, s, a);
-    } else {
-        hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, false, false, true>), dim3(blocks), dim3(256), 0, s, a);
+    if (a.eo) {
+        if (a.adjoint)
+            hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, false, true, true>), dim3(blocks), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, false, false, true>), dim3(blocks), dim3(256), 0, s, a);
+    } else if constexpr (NJ > 2 || RT == 128) {  // the others' columns fit diag_waves.hip's tiles
+        if (a.adjoint)
+            hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, false, true, false>), dim3(blocks), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((diag_modes_kernel<NJ, RT, true, false, false>), dim3(blocks), dim3(256), 0, s, a);
     }
     HZ_HIP(hipGetLastError());
     return HZ_OK;
@@ -69,6 +71,7 @@ int diag_tile_choices(int NP, int *rt, int max)
 
 int launch_diag_modes(const DiagArgs &a, hipStream_t s)
 {
+    if (!a.eo && diag_waves_holds(a.n, a.ne)) return launch_diag_waves(a, s);
     switch (diag_padded(a.n)) {
     case 32:
         return a.rt == 128 ? launch_t<2, 128>(a, s) : a.rt == 64 ? launch_t<2, 64>(a, s) : launch_t<2, 32>(a, s);

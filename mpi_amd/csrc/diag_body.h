@@ -166,6 +166,38 @@ __device__ __forceinline__ void tile_gemm(d4 (&acc)[RBK][JT], const double *tile
     }
 }
 
+// acc[rb] += A B for one column tile (column j of this lane), A = the LDS tile's
+// rows 16 rb + i (LD even, 16-byte aligned), B[k][j] = B[k * SB + j], k < NP.
+// Step 2 p + h runs over k = 8 p + 2 lk + h, so that one 16-byte LDS read holds
+// a lane's A operands of two steps; B four steps ahead.
+template <int NP, int LD, int RB, int SB = NP>
+__device__ __forceinline__ void pair_gemm(d4 (&acc)[RB], const double *tile, const double *__restrict__ B, int j,
+                                          int li, int lk)
+{
+    constexpr int NPR = NP / 8, D = 2;
+    const double *bc = B + 2 * lk * SB + j;
+    double b[D][2];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        b[d][0] = bc[8 * d * SB];
+        b[d][1] = bc[(8 * d + 1) * SB];
+    }
+#pragma unroll
+    for (int p = 0; p < NPR; ++p) {
+        const double v0 = b[p % D][0], v1 = b[p % D][1];
+        if (p + D < NPR) {
+            b[p % D][0] = bc[8 * (p + D) * SB];
+            b[p % D][1] = bc[(8 * (p + D) + 1) * SB];
+        }
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const double2 av = *reinterpret_cast<const double2 *>(tile + (16 * rb + li) * LD + 8 * p + 2 * lk);
+            acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, v0, acc[rb], 0, 0, 0);
+            acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, v1, acc[rb], 0, 0, 0);
+        }
+    }
+}
+
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef short s4 __attribute__((ext_vector_type(4)));
 

@@ -126,6 +126,10 @@ int diag_padded(int n);
 // Tile heights offered for padded size NP (autotuned per plan).
 int diag_tile_choices(int NP, int *rt, int max);
 int launch_diag_modes(const DiagArgs &a, hipStream_t s);
+// The same for several elements, Robin faces or periodic z at N - 2 <= 32
+// (diag_waves.hip); launch_diag_modes takes it where it holds.
+bool diag_waves_holds(int n, int ne);
+int launch_diag_waves(const DiagArgs &a, hipStream_t s);
 
 
 // The one-element Dirichlet solve with the z contractions outside the x-y

@@ -56,38 +56,8 @@ __global__ __launch_bounds__(256, 2) void mixed_modes_kernel(const MixedArgs a)
 // CU keep them busy for two thirds of the time, and 2,064 work-groups leave 16
 // for a fifth round.
 
-// acc += A B in FP64, step 2 p + h over rows k = 8 p + 2 lk + h; B's rows four
-// steps ahead.
-template <int NP, int LD, int RB>
-__device__ __forceinline__ void pair_gemm(d4 (&acc)[RB], const double *tile, const double *__restrict__ B, int j,
-                                          int li, int lk)
-{
-    constexpr int NPR = NP / 8, D = 2;
-    const double *bc = B + 2 * lk * NP + j;
-    double b[D][2];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        b[d][0] = bc[8 * d * NP];
-        b[d][1] = bc[(8 * d + 1) * NP];
-    }
-#pragma unroll
-    for (int p = 0; p < NPR; ++p) {
-        const double v0 = b[p % D][0], v1 = b[p % D][1];
-        if (p + D < NPR) {
-            b[p % D][0] = bc[8 * (p + D) * NP];
-            b[p % D][1] = bc[(8 * (p + D) + 1) * NP];
-        }
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const double2 av = *reinterpret_cast<const double2 *>(tile + (16 * rb + li) * LD + 8 * p + 2 * lk);
-            acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, v0, acc[rb], 0, 0, 0);
-            acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, v1, acc[rb], 0, 0, 0);
-        }
-    }
-}
-
 template <int NJ, int RB, bool GENERAL>
-__global__ __launch_bounds__(64 * NJ, 4) void mixed_waves_kernel(const MixedArgs a)
+__global__ __launch_bounds__(64 * NJ, NJ == 6 && GENERAL ? 3 : 4) void mixed_waves_kernel(const MixedArgs a)
 {
     constexpr int NP = 16 * NJ, H = NP / 2, RT = 16 * RB, T = 64 * NJ, KS = H / 4;
     constexpr int LD = NP + 2, LDF = NP + 4;      // conflict-free row strides

@@ -250,3 +250,43 @@ def test_mixed_one_wave_per_16_columns(cuda, N, faces, ne):
     h = plan.mixed_history()
     assert len(h) == 2 and 0 < h[1] < h[0] < 1e-3
     plan.close()
+
+
+@pytest.mark.parametrize("N,ne", [(3, 1), (4, 64), (9, 5), (17, 13), (18, 1), (18, 63), (19, 1), (19, 32), (33, 3),
+                                  (34, 7), (34, 31)])
+@pytest.mark.parametrize("faces", ["robin", "periodic", "dirichlet"])
+def test_diag_short_elements(cuda, N, ne, faces):
+    """The DIAG mode solve of several elements, Robin faces or periodic z at
+    N - 2 <= 32: 16 and 32 columns, whole and partial row tiles, up to the
+    largest element count of a tile.  Solve against the oracle within twice
+    its rounding spread (or 1e-12); adjoint by <S x, v> = <x, S^T v>."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    nx, ny, lam = 4, 8, 3.0
+    ab = (0.7, 1.3, 0.4, 2.0) if faces == "robin" else (0.0, 2.0, 0.0, -0.5)
+    geo = dict(xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2)
+    per = faces == "periodic"
+    kw = {} if per else dict(alpha_l=ab[0], beta_l=ab[1], alpha_r=ab[2], beta_r=ab[3])
+    plan = HelmholtzPlan(nx, ny, N, ne, lam=lam, form="diag", periodic_z=per, **geo, **kw)
+    r = np.random.default_rng(N + ne)
+    f = r.standard_normal((nx, ny, plan.nz))
+    g = [r.standard_normal((nx, ny)) for _ in range(2)]
+    dk = {} if per else dict(alphal=ab[0], betal=ab[1], alphar=ab[2], betar=ab[3])
+    desc = po.make_desc(nx, ny, ne * N, N, size=1, lam=lam, **geo, **dk)
+    df, dg = to_dev(f), [] if per else [to_dev(v) for v in g]
+    if per:
+        f[:, :, -1] = f[:, :, 0]
+        df = to_dev(f)
+        uo, uf = po.solve_periodic(desc, f), po.solve_periodic(desc, f, fma=True)
+    else:
+        uo, uf = po.solve(desc, f, *g), po.solve(desc, f, *g, fma=True)
+    u = plan.solve(df, *dg)
+    bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+    assert np.abs(u.cpu().numpy() - uo).max() <= bar * np.abs(uo).max()
+    v = to_dev(r.standard_normal(u.shape))
+    fbar, glbar, grbar, _ = plan.adjoint(v)
+    lhs = float((u * v).sum())
+    rhs = float((df * fbar).sum()) + (0.0 if per else float((dg[0] * glbar).sum() + (dg[1] * grbar).sum()))
+    scale = float((df * fbar).abs().sum() + (u * v).abs().sum())
+    assert abs(lhs - rhs) <= bar * scale
+    plan.close()
