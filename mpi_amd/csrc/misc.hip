@@ -10,20 +10,26 @@
 namespace hz {
 namespace {
 
-// Lanes are columns, a wave's registers hold kDerivRows output rows of 64
-// columns.  The column tile is staged in LDS (a lane's values one column
-// stride apart: the stride is odd, so 64 lanes hit different banks); the
-// matrix value of a step is the same in every lane, so it comes through the
-// scalar cache from the transposed copy DT[p][k] (KP = N rounded up to
-// kDerivRows).  One LDS read and kDerivRows products and sums a step, where a
-// thread per output node read a matrix row (uncoalesced) and a column from
-// the caches for every pair.  256^2 columns of N = 129: 2,727 -> 137 us; the
+// Lanes are columns, a wave's registers hold R output rows of 64 columns.  The
+// column tile is staged in LDS (a lane's values one column stride apart: the
+// stride is odd, so 64 lanes hit different banks) and takes the results for a
+// coalesced store; the matrix value of a step is the same in every lane, so it
+// comes through the scalar cache from the transposed copy DT[p][k] (KP = R
+// times the strips).  One LDS read and R products and sums a step, where a
+// thread per output node read a matrix row (uncoalesced) and a column from the
+// caches for every pair.  256^2 columns of N = 129: 2,727 -> 110 us (with strips of 16
+// rows and every lane storing its own rows 130); the
 // rounded products and sums cannot be fused, N^2 of each per column, which is
-// 55 us at one 16-lane operation per clock, and the rest is the scalar loads'
-// latency (the matrix, 149 KB, does not fit the scalar cache).
-constexpr int kDerivRows = 16;
+// 55 us at one 16-lane operation per clock.
+//
+// R = 17 where it saves a strip (N = 2^m + 1, the usual GLL sizes, would leave
+// one row to a strip of 16 that costs as much as the others, and an odd number
+// of waves to the four SIMDs).
 constexpr int kDerivCols = 64;
 
+int deriv_rows(int N) { return (N + 16) / 17 < (N + 15) / 16 ? 17 : 16; }
+
+template <int R>
 __global__ __launch_bounds__(1024) void derivative_kernel(const double *__restrict__ DT, int N, int KP, long long ncols,
                                                          const double *__restrict__ u, double *__restrict__ out)
 {
@@ -50,31 +56,32 @@ __global__ __launch_bounds__(1024) void derivative_kernel(const double *__restri
     }
     __syncthreads();
     const int lane = threadIdx.x % 64;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), waves = T / 64;
-    const double *uc = dtile + (lane < nc ? lane : 0) * LD;
-    for (int k0 = wave * kDerivRows; k0 < N; k0 += waves * kDerivRows) {
-        double acc[kDerivRows];
+    const int k0 = R * __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    double *uc = dtile + (lane < nc ? lane : 0) * LD;
+    double acc[R];
 #pragma unroll
-        for (int j = 0; j < kDerivRows; ++j) acc[j] = 0.0;
+    for (int j = 0; j < R; ++j) acc[j] = 0.0;
+    if (k0 < N) {
         const double *d = DT + k0;
 #pragma unroll 2
         for (int p = 0; p < N; ++p) {
             const double x = uc[p];
 #pragma unroll
-            for (int j = 0; j < kDerivRows; ++j) acc[j] += d[(long long)p * KP + j] * x;
+            for (int j = 0; j < R; ++j) acc[j] += d[(long long)p * KP + j] * x;
         }
-        if (lane < nc) {
-            double *o = out + (col0 + lane) * N + k0;
-            const int rows = N - k0 < kDerivRows ? N - k0 : kDerivRows;
-            if (rows == kDerivRows) {
+    }
+    __syncthreads();  // every wave has read the tile
+    if (lane < nc) {
 #pragma unroll
-                for (int j = 0; j < kDerivRows; ++j) o[j] = acc[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < kDerivRows; ++j)
-                    if (j < rows) o[j] = acc[j];
-            }
-        }
+        for (int j = 0; j < R; ++j)
+            if (k0 + j < N) uc[k0 + j] = acc[j];
+    }
+    __syncthreads();
+    double *dst = out + col0 * N;
+    if (LD == N) {
+        for (int i = threadIdx.x; i < total; i += T) dst[i] = dtile[i];
+    } else {
+        for (int i = threadIdx.x; i < total; i += T) dst[i] = dtile[i + i / N];
     }
 }
 
@@ -223,7 +230,7 @@ int launch_cubic_adjoint(const double *fbar, const double *u_in, const double *u
 
 std::vector<double> derivative_operand(const std::vector<double> &D, int N)
 {
-    const int KP = (N + kDerivRows - 1) / kDerivRows * kDerivRows;
+    const int R = deriv_rows(N), KP = (N + R - 1) / R * R;
     std::vector<double> t((size_t)N * KP, 0.0);
     for (int k = 0; k < N; ++k)
         for (int p = 0; p < N; ++p) t[(size_t)p * KP + k] = D[(size_t)k * N + p];
@@ -233,23 +240,25 @@ std::vector<double> derivative_operand(const std::vector<double> &D, int N)
 int derivative_prepare(int N)
 {
     const size_t lds = sizeof(double) * kDerivCols * (N | 1);
-    if (lds > 64 * 1024)
-        HZ_HIP(hipFuncSetAttribute((const void *)derivative_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   160 * 1024));
+    const void *f = deriv_rows(N) == 17 ? (const void *)derivative_kernel<17> : (const void *)derivative_kernel<16>;
+    if (lds > 64 * 1024) HZ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     return HZ_OK;
 }
 
 int launch_derivative(const double *DT, int N, long long ncols, const double *u, double *out, hipStream_t s)
 {
     if (ncols <= 0) return HZ_OK;
-    const int strips = (N + kDerivRows - 1) / kDerivRows;
-    // one strip per wave, at most 16 waves (evenly filled passes above)
-    const int passes = (strips + 15) / 16, waves = std::max(2, (strips + passes - 1) / passes);
+    // one strip per wave
+    const int R = deriv_rows(N), strips = (N + R - 1) / R, waves = std::max(2, strips);
     const size_t lds = sizeof(double) * kDerivCols * (N | 1);
     const long long blocks = (ncols + kDerivCols - 1) / kDerivCols;
-    if (lds > 160 * 1024 || blocks > 0x7fffffffLL) return set_error(HZ_ERR_UNSUPPORTED, "derivative: field too large");
-    hipLaunchKernelGGL(derivative_kernel, dim3((unsigned)blocks), dim3(64 * waves), (unsigned)lds, s, DT, N,
-                       strips * kDerivRows, ncols, u, out);
+    if (waves > 16 || lds > 160 * 1024 || blocks > 0x7fffffffLL)
+        return set_error(HZ_ERR_UNSUPPORTED, "derivative: field too large");
+    const dim3 grid((unsigned)blocks), block(64 * waves);
+    if (R == 17)
+        hipLaunchKernelGGL((derivative_kernel<17>), grid, block, (unsigned)lds, s, DT, N, strips * R, ncols, u, out);
+    else
+        hipLaunchKernelGGL((derivative_kernel<16>), grid, block, (unsigned)lds, s, DT, N, strips * R, ncols, u, out);
     HZ_HIP(hipGetLastError());
     return HZ_OK;
 }
