@@ -17,6 +17,10 @@
 // launch API checks that every work-group is resident, and every work-group
 // runs the same stage loop, so each barrier is reached by all of them.
 //
+// One-element Dirichlet problems in DIAG form leave this scheme where the
+// z-first kernels (zfirst.hip) hold them: three stages of lists, launched ahead
+// of the rest in every variant.
+//
 // The autotuner times the usable variants (staged or fused, mode-solve tile
 // height 32 or 64 rows) on the first solve of a batch shape and keeps the
 // fastest.
@@ -317,6 +321,10 @@ using namespace hz;
 // ---- host side ---------------------------------------------------------------
 namespace {
 
+// One element with Dirichlet faces in DIAG form, and a grid of the z-first
+// kernels (zfirst.hip): expand, filter, collect instead of the five stages.
+bool z_first(const hz_plan *pl) { return pl->d.form == HZ_FORM_DIAG && pl->zf && !diag_general(pl); }
+
 struct Variant {
     int rt;           // diag tile rows
     int fused;        // 1 one launch for the whole batch, 0 one launch per stage and task kind,
@@ -363,6 +371,12 @@ struct hz_batch {
     std::vector<int> h_coop_off[2];  // host copy (the merged variant's launch sizes)
     int *d_ctr = nullptr;
     int coop_wgs[2] = {0, 0};
+    // z-first problems: their arguments (one entry per problem of the batch),
+    // tiles and launches {stage, kind, first, count}
+    ZfArgs *d_zargs = nullptr, *h_zargs = nullptr;
+    int2 *d_zlist = nullptr;
+    std::vector<std::array<int, 4>> zlaunches;
+    bool zuse = false;
     std::vector<const void *> last;
     std::vector<unsigned> gens;  // each plan's generation when the tables were built
     std::string shape;
@@ -402,6 +416,7 @@ int fill_problems(hz_batch *b, const double *const *f, const double *const *gl, 
                               nullptr, xs);
         q.f[3] = xy_pass_args(pl, 3, nullptr, pl->spec.re, pl->spec.im, u[p], pl->K, nullptr, nullptr, nullptr,
                               nullptr, xs);
+        if (z_first(pl)) b->h_zargs[p] = zf_args(pl, f[p], u[p], gl[p], gr[p]);
         if (pl->d.form == HZ_FORM_MIXED)
             q.m = mixed_args(pl);
         else
@@ -472,6 +487,8 @@ template <int RT>
 int enqueue_t(hz_batch *b, const Variant &v, hipStream_t s)
 {
     const int r = rt_index(RT);
+    for (const auto &z : b->zlaunches)
+        if (int st = launch_zf_list(b->d_zargs, b->d_zlist + z[2], z[3], z[0], z[1], s)) return st;
     if (v.fused == 2) {
         const auto &xo = b->h_coop_off[r];
         for (int st = 0; st < kStages; ++st) {
@@ -523,6 +540,49 @@ int enqueue_t(hz_batch *b, const Variant &v, hipStream_t s)
     return HZ_OK;
 }
 
+// Tiles of the z-first problems, by stage and kind: 64 problems of 32 to 128
+// points a side and 17 to 129 along z (317 MB) take 400 us, 600 in five stages.
+// Used from one tile per CU on (16 of 32 x 32 x 17: 78 us either way; x 129 80
+// against 96): on fewer, the five stages' many short work-groups fill the chip
+// better.
+int build_zlists(hz_batch *b)
+{
+    int tiles = 0;
+    for (const hz_plan *pl : b->plans)
+        if (z_first(pl)) tiles += pl->nx * pl->ny / 64;
+    b->zuse = tiles >= b->cus;
+    b->zlaunches.clear();
+    (void)hipFree(b->d_zlist);
+    b->d_zlist = nullptr;
+    if (!b->zuse) return HZ_OK;
+    // {stage, launch kind} -> size -> tiles.  Within a launch, XCD x's range
+    // holds the x-th eighth of every size, the larger ones first: even shares,
+    // and neighbouring work-groups run the same code.
+    std::map<std::pair<int, int>, std::map<int, std::vector<int2>>> by;
+    for (int p = 0; p < b->n; ++p) {
+        const hz_plan *pl = b->plans[p];
+        if (!z_first(pl)) continue;
+        for (int st = 0; st < 3; ++st) {
+            auto &v = by[{st, zf_kind(pl->nx, pl->ny, pl->n, st)}][st == 1 ? -(pl->nx * 1024 + pl->ny) : -pl->NP];
+            for (int t = 0, nt = zf_tasks(pl->nx, pl->ny, pl->n, st); t < nt; ++t) v.push_back(make_int2(p, t));
+        }
+    }
+    std::vector<int2> all;
+    for (auto &kv : by) {
+        const size_t first = all.size();
+        for (int x = 0; x < kXcds; ++x)
+            for (auto &sz : kv.second) {
+                const auto &v = sz.second;
+                all.insert(all.end(), v.begin() + v.size() * x / kXcds, v.begin() + v.size() * (x + 1) / kXcds);
+            }
+        b->zlaunches.push_back({kv.first.first, kv.first.second, (int)first, (int)(all.size() - first)});
+    }
+    if (hipMalloc((void **)&b->d_zlist, sizeof(int2) * all.size()) != hipSuccess)
+        return set_error(HZ_ERR_ALLOC, "batch allocation failed");
+    HZ_HIP(hipMemcpy(b->d_zlist, all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice));
+    return HZ_OK;
+}
+
 // Task lists of the staged variant for tile height rt (problem kinds known
 // from the filled problem table).
 int build_lists(hz_batch *b, int rt)
@@ -531,6 +591,7 @@ int build_lists(hz_batch *b, int rt)
     std::map<std::pair<int, int>, std::vector<int2>> by;
     for (int p = 0; p < b->n; ++p)
         for (int st = 0; st < kStages; ++st) {
+            if (b->zuse && z_first(b->plans[p])) continue;
             auto &v = by[{st, task_kind(b->h_probs[p], st)}];
             int ntask = st == 2 ? mode_tiles(b->plans[p], rt) : 0;
             if (st != 2) {  // transform passes: one entry per uniform-base tile
@@ -566,7 +627,8 @@ int build_lists(hz_batch *b, int rt)
     b->groups[r].push_back({kStages, 0, (int)all.size()});
     (void)hipFree(b->d_list[r]);
     b->d_list[r] = nullptr;
-    if (hipMalloc((void **)&b->d_list[r], sizeof(int2) * all.size()) != hipSuccess)
+    // (one entry more: a batch of z-first problems only has none)
+    if (hipMalloc((void **)&b->d_list[r], sizeof(int2) * (all.size() + 1)) != hipSuccess)
         return set_error(HZ_ERR_ALLOC, "batch allocation failed");
     HZ_HIP(hipMemcpy(b->d_list[r], all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice));
     // The fused variant's order: within each stage, XCD x's range holds the
@@ -593,7 +655,7 @@ int build_lists(hz_batch *b, int rt)
     (void)hipFree(b->d_coop_off[r]);
     b->d_coop_list[r] = nullptr;
     b->d_coop_off[r] = nullptr;
-    if (hipMalloc((void **)&b->d_coop_list[r], sizeof(int2) * co.size()) != hipSuccess ||
+    if (hipMalloc((void **)&b->d_coop_list[r], sizeof(int2) * (co.size() + 1)) != hipSuccess ||
         hipMalloc((void **)&b->d_coop_off[r], sizeof(int) * xo.size()) != hipSuccess)
         return set_error(HZ_ERR_ALLOC, "batch allocation failed");
     HZ_HIP(hipMemcpy(b->d_coop_list[r], co.data(), sizeof(int2) * co.size(), hipMemcpyHostToDevice));
@@ -615,6 +677,7 @@ int upload_problems(hz_batch *b, const double *const *f, const double *const *gl
     HZ_HIP(hipStreamSynchronize(b->stream));  // the pinned table may still be in flight
     fill_problems(b, f, gl, gr, u);
     HZ_HIP(hipMemcpyAsync(b->d_probs, b->h_probs, sizeof(BatchProblem) * b->n, hipMemcpyHostToDevice, b->stream));
+    HZ_HIP(hipMemcpyAsync(b->d_zargs, b->h_zargs, sizeof(ZfArgs) * b->n, hipMemcpyHostToDevice, b->stream));
     return HZ_OK;
 }
 
@@ -639,6 +702,7 @@ int rebuild_lists(hz_batch *b)
 {
     std::vector<const double *> nil(b->n, nullptr);
     std::vector<double *> nilo(b->n, nullptr);
+    if (int st = build_zlists(b)) return st;
     for (int r = 0; r < 2; ++r) {
         fill_problems(b, nil.data(), nil.data(), nil.data(), nilo.data());
         if (int st = build_lists(b, r ? 64 : 32)) return st;
@@ -687,6 +751,9 @@ void free_batch(hz_batch *b)
     if (b->stream) (void)hipStreamDestroy(b->stream);
     (void)hipFree(b->d_probs);
     (void)hipHostFree(b->h_probs);
+    (void)hipFree(b->d_zargs);
+    (void)hipHostFree(b->h_zargs);
+    (void)hipFree(b->d_zlist);
     for (int2 *l : b->d_list) (void)hipFree(l);
     for (int2 *l : b->d_coop_list) (void)hipFree(l);
     for (int *o : b->d_coop_off) (void)hipFree(o);
@@ -737,6 +804,8 @@ int hz_batch_create(hz_plan *const *plans, int count, hz_batch **batch)
         return fail(set_error(HZ_ERR_HIP, "stream/event creation failed"));
     if (hipMalloc((void **)&b->d_probs, sizeof(BatchProblem) * count) != hipSuccess ||
         hipHostMalloc((void **)&b->h_probs, sizeof(BatchProblem) * count) != hipSuccess ||
+        hipMalloc((void **)&b->d_zargs, sizeof(ZfArgs) * count) != hipSuccess ||
+        hipHostMalloc((void **)&b->h_zargs, sizeof(ZfArgs) * count) != hipSuccess ||
         hipMalloc((void **)&b->d_ctl, sizeof(int) * 4) != hipSuccess ||
         hipMalloc((void **)&b->d_ctr, sizeof(int) * kStages * kXcds) != hipSuccess)
         return fail(set_error(HZ_ERR_ALLOC, "batch allocation failed"));

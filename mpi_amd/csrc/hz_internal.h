@@ -154,8 +154,15 @@ struct ZfArgs {
     int adjoint, cubic;
     double c3, c1;              // cubic: the right-hand side f (c3 f^2 + c1)
 };
-bool zf_holds(int nx, int ny, int n);
+bool zf_holds(int nx, int ny, int n);  // where one solve is faster this way
 int launch_zf(const ZfArgs &a, int stage, hipStream_t s);
+// The forward stages over many problems: every grid of zf_fits; work-group i
+// takes tile list[i].y of problem Z[list[i].x], the entries of one launch being
+// of one zf_kind; a problem has zf_tasks tiles.
+bool zf_fits(int nx, int ny, int n);
+int zf_kind(int nx, int ny, int n, int stage);
+int zf_tasks(int nx, int ny, int n, int stage);
+int launch_zf_list(const ZfArgs *Z, const int2 *list, int count, int stage, int kind, hipStream_t s);
 
 // MIXED form (mixed.hip, mixed_body.h): FP32 eigenbasis solves refined with
 // FP64 residuals, both on the matrix cores.
@@ -253,6 +260,8 @@ bool diag_general(const hz_plan *p);  // several elements, Robin faces or period
 void diag_basis(const hz_plan *p, DiagArgs &a, bool adjoint);
 // Arguments of the MIXED mode solve on `p`'s workspace.
 MixedArgs mixed_args(const hz_plan *p);
+// Arguments of the z-first forward solve on `p`'s workspace.
+ZfArgs zf_args(const hz_plan *p, const double *f, double *u, const double *gl, const double *gr);
 }  // namespace hz
 
 // ---- the plan ----------------------------------------------------------------
@@ -289,10 +298,11 @@ struct hz_plan {
     double *d_eo_vec = nullptr, *d_eo_B1 = nullptr, *d_eo_B2 = nullptr, *d_eo_hom = nullptr;
     double *d_eo_B1a = nullptr, *d_eo_B2a = nullptr;  // adjoint operands
     short *d_eo_M = nullptr, *d_eo_Ma = nullptr;      // first-order correction (bf16), forward and adjoint
-    // z-first solve (zfirst.hip), where it applies: the operands in one
+    // z-first solve (zfirst.hip), where it applies (zf_route: and is faster for
+    // one solve alone): the operands in one
     // allocation (forward B1, B2, X1, X2, then the adjoint's; w0, wN, mu), the
     // bf16 corrections in another, and the shifts' two parts
-    bool zf = false;
+    bool zf = false, zf_route = false;
     double *d_zf = nullptr, *d_zf_shift = nullptr;
     short *d_zf_C = nullptr;
     int diag_rt = 0;                                  // autotuned tile rows

@@ -251,7 +251,7 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
     static std::map<std::pair<std::vector<double>, int>, std::array<std::vector<short>, 2>> cache_m;
     static std::map<std::pair<std::vector<double>, int>, ZfOperands> cache_zf;
     // one element, Dirichlet faces, and a grid that the z-first kernels hold
-    const bool zf = zf_holds(p->nx, p->ny, n) && !diag_general(p);
+    const bool zf = zf_fits(p->nx, p->ny, n) && !diag_general(p);
     ZfOperands zo;
     std::vector<double> mu, W, Wi;
     std::array<std::vector<short>, 2> Mq;
@@ -350,6 +350,7 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
             (st = dmalloc(&p->d_zf_shift, (size_t)p->nx / 2 + 1 + p->M)))
             return st;
         p->zf = true;
+        p->zf_route = zf_holds(p->nx, p->ny, n);
     }
     return HZ_OK;
 }
@@ -572,6 +573,48 @@ int setup_diag(hz_plan *p)
 }
 
 }  // namespace
+
+static ZfArgs zf_args_any(const hz_plan *p, bool adjoint, const double *f, double *u)
+{
+    const size_t Q = (size_t)p->NP * p->NP, set = 2 * Q + 1024 + 2 * p->NP;
+    const double *d = p->d_zf + (adjoint ? set : 0);
+    const short *c = p->d_zf_C + (adjoint ? 2 * Q : 0);
+    ZfArgs a{};
+    a.nx = p->nx;
+    a.ny = p->ny;
+    a.K = p->K;
+    a.n = p->n;
+    while ((16 << a.lr2) < p->ny) ++a.lr2;
+    a.ncol = p->nx << a.lr2;
+    a.f = f;
+    a.u = u;
+    a.beta_l = p->d.beta_l;
+    a.beta_r = p->d.beta_r;
+    a.T = p->spec.re;
+    a.B1 = d;
+    a.B2 = d + Q;
+    a.X1 = d + 2 * Q;
+    a.X2 = a.X1 + 512;
+    a.w0 = a.X2 + 512;
+    a.wN = a.w0 + p->NP;
+    a.C1 = c;
+    a.C2 = c + Q;
+    a.mu = p->d_zf + 2 * set;
+    a.sx = p->d_zf_shift;
+    a.sy = p->d_zf_shift + p->nx / 2 + 1;
+    a.twx = p->d_twx;
+    a.twy = p->d_twy;
+    a.adjoint = adjoint;
+    return a;
+}
+
+ZfArgs hz::zf_args(const hz_plan *p, const double *f, double *u, const double *gl, const double *gr)
+{
+    ZfArgs a = zf_args_any(p, false, f, u);
+    a.gl = gl;
+    a.gr = gr;
+    return a;
+}
 
 // Arguments of the MIXED mode solve on `p`'s workspace.
 MixedArgs hz::mixed_args(const hz_plan *p)
@@ -1187,40 +1230,11 @@ int hz_plan_set_robin(hz_plan *p, double alpha_l, double beta_l, double alpha_r,
 static int zf_pipeline(hz_plan *p, const double *f, double *u, const double *gl, const double *gr, double *glbar,
                        double *grbar, const double *cubic, hipStream_t s, StageRecorder *rec)
 {
-    const size_t Q = (size_t)p->NP * p->NP, set = 2 * Q + 1024 + 2 * p->NP;
-    const bool adj = glbar != nullptr;
-    const double *d = p->d_zf + (adj ? set : 0);
-    const short *c = p->d_zf_C + (adj ? 2 * Q : 0);
-    ZfArgs a{};
-    a.nx = p->nx;
-    a.ny = p->ny;
-    a.K = p->K;
-    a.n = p->n;
-    while ((16 << a.lr2) < p->ny) ++a.lr2;
-    a.ncol = p->nx << a.lr2;
-    a.f = f;
-    a.u = u;
+    ZfArgs a = zf_args_any(p, glbar != nullptr, f, u);
     a.gl = gl;
     a.gr = gr;
     a.glbar = glbar;
     a.grbar = grbar;
-    a.beta_l = p->d.beta_l;
-    a.beta_r = p->d.beta_r;
-    a.T = p->spec.re;
-    a.B1 = d;
-    a.B2 = d + Q;
-    a.X1 = d + 2 * Q;
-    a.X2 = a.X1 + 512;
-    a.w0 = a.X2 + 512;
-    a.wN = a.w0 + p->NP;
-    a.C1 = c;
-    a.C2 = c + Q;
-    a.mu = p->d_zf + 2 * set;
-    a.sx = p->d_zf_shift;
-    a.sy = p->d_zf_shift + p->nx / 2 + 1;
-    a.twx = p->d_twx;
-    a.twy = p->d_twy;
-    a.adjoint = adj;
     if (cubic) {
         a.cubic = 1;
         a.c3 = cubic[0];
@@ -1245,7 +1259,7 @@ static int solve_impl(hz_plan *p, const double *f, const double *gl, const doubl
         return set_error(HZ_ERR_ARG, "null face data");
     }
     StageRecorder rec(p, s);
-    if (p->d.form == HZ_FORM_DIAG && p->zf && !diag_general(p) && !op_diag && !op_full)
+    if (p->d.form == HZ_FORM_DIAG && p->zf_route && !diag_general(p) && !op_diag && !op_full)
         return zf_pipeline(p, f, u, gl, gr, nullptr, nullptr, cubic, s, &rec);
     int st = forward_xy(p, f, p->spec.re, p->spec.im, p->K, s, gl, gr, p->xs, cubic);
     rec.mark("fft_forward");
@@ -1360,7 +1374,7 @@ static int adjoint_pipeline(hz_plan *p, const double *ubar, double *fbar, double
                             hipStream_t s, StageRecorder *rec)
 {
     int st;
-    if (p->zf && !diag_general(p)) return zf_pipeline(p, ubar, fbar, nullptr, nullptr, glbar, grbar, nullptr, s, rec);
+    if (p->zf_route && !diag_general(p)) return zf_pipeline(p, ubar, fbar, nullptr, nullptr, glbar, grbar, nullptr, s, rec);
     if ((st = forward_xy(p, ubar, p->spec.re, p->spec.im, p->K, s, nullptr, nullptr, p->xs))) return st;
     if (rec) rec->mark("fft_forward");
     DiagArgs a = diag_args(p);

@@ -190,6 +190,13 @@ struct CorrLds {
                                                                               : kRows * (16 * NJ + 2);
 };
 
+// LDS of one tile of an end kernel.
+template <int NJ>
+struct alignas(16) EndLds {
+    double tile[CorrLds<NJ>::DOUBLES];
+    double rows[2][kRows];
+};
+
 template <int NJ>
 __device__ __forceinline__ void to_corr(const d4 (&acc)[4][1], double *tile, int w, int li, int lk)
 {
@@ -266,14 +273,12 @@ __device__ __forceinline__ int compact(int j, int he, int ho)
 // share a CU), correction (20%) and stores hardly overlap: without the loads
 // 41 us, without the contraction 33, without the stores 44.
 template <int NJ, bool ADJ, bool CUB>
-__global__ __launch_bounds__(64 * NJ, 4) void zf_expand(const ZfArgs a)
+__device__ __forceinline__ void expand_tile(const ZfArgs &a, int c0, int tid, EndLds<NJ> &lds)
 {
     constexpr int NP = 16 * NJ, LD = NP + 2, H = NP / 2, T = 64 * NJ;
-    __shared__ alignas(16) double tile[CorrLds<NJ>::DOUBLES];
-    __shared__ double row_zl[kRows], row_zr[kRows];
-    const int tid = threadIdx.x, lane = tid % 64, w = uniform(tid / 64), li = lane % 16, lk = lane / 16;
+    double *tile = lds.tile, *row_zl = lds.rows[0], *row_zr = lds.rows[1];
+    const int lane = tid % 64, w = uniform(tid / 64), li = lane % 16, lk = lane / 16;
     const int n = a.n, ho = n / 2, he = n - ho;
-    const int c0 = 4 * xcd_logical(blockIdx.x, gridDim.x);
     if constexpr (!ADJ) {
         if (tid < kRows) {
             const RowAt at(tid, c0, a.lr2);
@@ -339,14 +344,13 @@ __global__ __launch_bounds__(64 * NJ, 4) void zf_expand(const ZfArgs a)
 // ---- 3: 16-point stage back, correction, contraction, store --------------------
 // zf_expand's mirror image and bounds; 256^2 x 129: 55 us (adjoint 57).
 template <int NJ, bool ADJ>
-__global__ __launch_bounds__(64 * NJ, NJ == 6 ? 3 : 4) void zf_collect(const ZfArgs a)
+__device__ __forceinline__ void collect_tile(const ZfArgs &a, int c0, int tid, EndLds<NJ> &lds)
 {
     constexpr int NP = 16 * NJ, LD = NP + 2, H = NP / 2, T = 64 * NJ;
-    __shared__ alignas(16) double tile[CorrLds<NJ>::DOUBLES];
-    __shared__ double face[2][ADJ ? kRows : 1];
-    const int tid = threadIdx.x, lane = tid % 64, w = uniform(tid / 64), li = lane % 16, lk = lane / 16;
+    double *tile = lds.tile;
+    auto &face = lds.rows;
+    const int lane = tid % 64, w = uniform(tid / 64), li = lane % 16, lk = lane / 16;
     const int n = a.n, ho = n / 2, he = n - ho;
-    const int c0 = 4 * xcd_logical(blockIdx.x, gridDim.x);
     const int jc = compact<H>(16 * w + li, he, ho);
     d4 acc[4][1];
     {
@@ -435,6 +439,96 @@ __global__ __launch_bounds__(64 * NJ, NJ == 6 ? 3 : 4) void zf_collect(const ZfA
     }
 }
 
+template <int NJ, bool ADJ, bool CUB>
+__global__ __launch_bounds__(64 * NJ, 4) void zf_expand(const ZfArgs a)
+{
+    __shared__ EndLds<NJ> lds;
+    expand_tile<NJ, ADJ, CUB>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
+}
+
+template <int NJ, bool ADJ>
+__global__ __launch_bounds__(64 * NJ, NJ == 6 ? 3 : 4) void zf_collect(const ZfArgs a)
+{
+    __shared__ EndLds<NJ> lds;
+    collect_tile<NJ, ADJ>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
+}
+
+// Many problems: one (problem, tile) entry per work-group.  Pointers read from
+// memory are marked as global ones (as kernel arguments are): generic loads
+// would wait on the LDS counter as well and cost the filter 100 registers.
+template <class V>
+__device__ __forceinline__ V *as_global(V *p)
+{
+    return (V *)(V __attribute__((address_space(1))) *)sval((unsigned long long)p);
+}
+__device__ __forceinline__ ZfArgs problem_args(const ZfArgs *__restrict__ Z, int p)
+{
+    ZfArgs a = Z[p];
+    a.nx = uniform(a.nx);
+    a.ny = uniform(a.ny);
+    a.n = uniform(a.n);
+    a.K = uniform(a.K);
+    a.lr2 = uniform(a.lr2);
+    a.ncol = uniform(a.ncol);
+    a.f = as_global(a.f);
+    a.u = as_global(a.u);
+    a.gl = as_global(a.gl);
+    a.gr = as_global(a.gr);
+    a.T = as_global(a.T);
+    a.B1 = as_global(a.B1);
+    a.B2 = as_global(a.B2);
+    a.C1 = as_global(a.C1);
+    a.C2 = as_global(a.C2);
+    a.X1 = as_global(a.X1);
+    a.X2 = as_global(a.X2);
+    a.w0 = as_global(a.w0);
+    a.wN = as_global(a.wN);
+    a.mu = as_global(a.mu);
+    a.sx = as_global(a.sx);
+    a.sy = as_global(a.sy);
+    a.twx = as_global(a.twx);
+    a.twy = as_global(a.twy);
+    return a;
+}
+
+// Tiles of a work-group of 512 threads: as many as its threads and the LDS of
+// one of the widest hold.
+__host__ __device__ constexpr int end_tiles(int NJ) { return NJ >= 6 ? 1 : NJ == 4 ? 2 : 3; }
+
+template <int NJ, bool COLLECT>
+__device__ __forceinline__ void end_tiles_of(const ZfArgs &a, int task, char *smem)
+{
+    asm volatile("" ::: "memory");  // nothing of one size's body is formed ahead of the choice
+    constexpr int T = 64 * NJ, PER = end_tiles(NJ);
+    const int sub = uniform(threadIdx.x / T), t = task * PER + sub;
+    if (sub >= PER || 4 * t >= a.ncol) return;  // waves that ended take no part in the barriers
+    EndLds<NJ> &lds = reinterpret_cast<EndLds<NJ> *>(smem)[sub];
+    if constexpr (COLLECT)
+        collect_tile<NJ, false>(a, 4 * t, threadIdx.x % T, lds);
+    else
+        expand_tile<NJ, false, false>(a, 4 * t, threadIdx.x % T, lds);
+}
+
+// Every problem of a batch in one launch: its tasks of different sizes fill the
+// chip together, where a launch per size leaves most of it idle for the 10 to
+// 20 us that one work-group takes (64 problems, 317 MB: expand 130 us against
+// 147 in four launches, collect 140 against 169).
+template <bool COLLECT>
+__global__ __launch_bounds__(512, 4) void zf_end_list(const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
+{
+    __shared__ alignas(16) char smem[2 * sizeof(EndLds<4>)];
+    static_assert(sizeof(smem) >= sizeof(EndLds<8>) && sizeof(smem) >= 3 * sizeof(EndLds<2>), "every size fits");
+    const int2 e = list[xcd_logical(blockIdx.x, gridDim.x)];
+    const ZfArgs a = problem_args(Z, uniform(e.x));
+    const int task = uniform(e.y);
+    switch ((a.n + 31) / 32) {
+    case 1: end_tiles_of<2, COLLECT>(a, task, smem); break;
+    case 2: end_tiles_of<4, COLLECT>(a, task, smem); break;
+    case 3: end_tiles_of<6, COLLECT>(a, task, smem); break;
+    default: end_tiles_of<8, COLLECT>(a, task, smem); break;
+    }
+}
+
 // ---- 2: the rest of the transforms and the filter ------------------------------
 // One (j, k1) block of NX x R2 points per group of threads, 16 points per
 // thread in every stage: x in two register stages (NX = RA RB), the remaining
@@ -450,20 +544,19 @@ struct Filter {
     static constexpr int T = CH >= 4096 ? 256 : CH >= 2048 ? 128 : 64;
     static constexpr int NCH = 16 * T / CH;           // blocks per work-group
     static constexpr int LR = R2 + 1;
-    // 16-point stages in both directions take 162 registers: bounded to 128
-    // they spill 144 bytes a thread (45 us against 38 at 256^2 x 129)
-    static constexpr int WAVES = T == 256 ? 3 : 4;
+    // 16-point stages along y in both directions take 162 registers: bounded to
+    // 128 they spill 144 bytes a thread (45 us against 38 at 256^2 x 129)
+    static constexpr int WAVES = R2 == 16 ? 3 : 4;
+    static constexpr int LDS = NCH * NX * LR;         // doubles
     static_assert(NCH >= 1, "a block fits a work-group");
 };
 
 template <int NX, int R2>
-__global__ __launch_bounds__((Filter<NX, R2>::T), (Filter<NX, R2>::WAVES)) void zf_filter(const ZfArgs a)
+__device__ __forceinline__ void filter_tile(const ZfArgs &a, int wg, double *tile)
 {
     using S = Filter<NX, R2>;
     constexpr int RA = S::RA, RB = S::RB, NY = S::NY, CH = S::CH, T = S::T, NCH = S::NCH, LR = S::LR;
-    __shared__ double tile[NCH * NX * LR];
     const int tid = threadIdx.x;
-    const int wg = xcd_logical(blockIdx.x, gridDim.x);
     const int tasks = 9 * a.n;
     // item -> its block in the work-group (of IPB items each) and the rest
     auto block_of = [](int it, int ipb) { return NCH == 1 ? 0 : it / ipb; };
@@ -613,6 +706,55 @@ __global__ __launch_bounds__((Filter<NX, R2>::T), (Filter<NX, R2>::WAVES)) void 
     }
 }
 
+template <int NX, int R2>
+__global__ __launch_bounds__((Filter<NX, R2>::T), (Filter<NX, R2>::WAVES)) void zf_filter(const ZfArgs a)
+{
+    __shared__ double tile[Filter<NX, R2>::LDS];
+    filter_tile<NX, R2>(a, xcd_logical(blockIdx.x, gridDim.x), tile);
+}
+
+template <int NX, int R2>
+__device__ __forceinline__ void filter_of(const ZfArgs &a, int task, double *tile)
+{
+    asm volatile("" ::: "memory");  // nothing of one grid's body is formed ahead of the choice
+    filter_tile<NX, R2>(a, task, tile);
+}
+
+// The grids of a batch whose work-groups are one wave (R2 < 16), one launch: 73
+// us for 64 problems (317 MB) against 157 in nine; bounded to 128 registers it
+// spills and takes 117.
+constexpr int kFilterLds = 16 * 32 * 3;  // doubles: 32 x 2 pads most
+__global__ __launch_bounds__(64, 3) void zf_filter_list64(const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
+{
+    __shared__ double tile[kFilterLds];
+    const int2 e = list[xcd_logical(blockIdx.x, gridDim.x)];
+    const ZfArgs a = problem_args(Z, uniform(e.x));
+    const int task = uniform(e.y);
+    switch (a.nx * 1024 + a.ny) {
+    case 32 * 1024 + 32: filter_of<32, 2>(a, task, tile); break;
+    case 32 * 1024 + 64: filter_of<32, 4>(a, task, tile); break;
+    case 32 * 1024 + 128: filter_of<32, 8>(a, task, tile); break;
+    case 64 * 1024 + 32: filter_of<64, 2>(a, task, tile); break;
+    case 64 * 1024 + 64: filter_of<64, 4>(a, task, tile); break;
+    case 64 * 1024 + 128: filter_of<64, 8>(a, task, tile); break;
+    case 128 * 1024 + 32: filter_of<128, 2>(a, task, tile); break;
+    case 128 * 1024 + 64: filter_of<128, 4>(a, task, tile); break;
+    case 128 * 1024 + 128: filter_of<128, 8>(a, task, tile); break;
+    case 256 * 1024 + 32: filter_of<256, 2>(a, task, tile); break;
+    default: filter_of<256, 4>(a, task, tile); break;
+    }
+}
+
+// A larger grid of a batch.
+template <int NX, int R2>
+__global__ __launch_bounds__((Filter<NX, R2>::T), (Filter<NX, R2>::WAVES)) void zf_filter_list(
+    const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
+{
+    __shared__ double tile[Filter<NX, R2>::LDS];
+    const int2 e = list[xcd_logical(blockIdx.x, gridDim.x)];
+    filter_tile<NX, R2>(problem_args(Z, uniform(e.x)), uniform(e.y), tile);
+}
+
 template <int NJ>
 int launch_ends(const ZfArgs &a, bool collect, hipStream_t s)
 {
@@ -682,6 +824,52 @@ bool zf_holds(int nx, int ny, int n)
 {
     if (nx < 64 || nx > 256 || ny < 32 || ny > 256 || n < 1 || n > 128) return false;
     return nx * ny >= 16384 || (nx * ny >= 8192 && n >= 64);
+}
+
+bool zf_fits(int nx, int ny, int n)
+{
+    return nx >= 32 && nx <= 256 && ny >= 32 && ny <= 256 && n >= 1 && n <= 128;
+}
+
+int zf_kind(int nx, int ny, int n, int stage)
+{
+    const int grid = nx * 1024 + ny;
+    return stage != 1 || (nx * ny <= 16384 && ny < 256) ? 0 : grid;
+}
+
+int zf_tasks(int nx, int ny, int n, int stage)
+{
+    if (stage != 1) {
+        const int per = end_tiles(diag_padded(n) / 16);
+        return (nx * ny / 64 + per - 1) / per;
+    }
+    const int points = nx * ny / 16, blocks = points >= 1024 ? 1 : 1024 / points;  // Filter::CH, NCH
+    return (9 * n + blocks - 1) / blocks;
+}
+
+template <int NX, int R2>
+static void launch_filter_list(const ZfArgs *Z, const int2 *list, int count, hipStream_t s)
+{
+    hipLaunchKernelGGL((zf_filter_list<NX, R2>), dim3(count), dim3(Filter<NX, R2>::T), 0, s, Z, list);
+}
+
+int launch_zf_list(const ZfArgs *Z, const int2 *list, int count, int stage, int kind, hipStream_t s)
+{
+    if (stage == 0)
+        hipLaunchKernelGGL(zf_end_list<false>, dim3(count), dim3(512), 0, s, Z, list);
+    else if (stage == 2)
+        hipLaunchKernelGGL(zf_end_list<true>, dim3(count), dim3(512), 0, s, Z, list);
+    else
+        switch (kind) {
+        case 0: hipLaunchKernelGGL(zf_filter_list64, dim3(count), dim3(64), 0, s, Z, list); break;
+        case 32 * 1024 + 256: launch_filter_list<32, 16>(Z, list, count, s); break;
+        case 64 * 1024 + 256: launch_filter_list<64, 16>(Z, list, count, s); break;
+        case 128 * 1024 + 256: launch_filter_list<128, 16>(Z, list, count, s); break;
+        case 256 * 1024 + 128: launch_filter_list<256, 8>(Z, list, count, s); break;
+        default: launch_filter_list<256, 16>(Z, list, count, s); break;
+        }
+    HZ_HIP(hipGetLastError());
+    return HZ_OK;
 }
 
 int launch_zf(const ZfArgs &a, int stage, hipStream_t s)

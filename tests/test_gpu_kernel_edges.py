@@ -290,3 +290,41 @@ def test_diag_short_elements(cuda, N, ne, faces):
     scale = float((df * fbar).abs().sum() + (u * v).abs().sum())
     assert abs(lhs - rhs) <= bar * scale
     plan.close()
+
+
+def test_batch_z_first_every_grid(cuda):
+    """The z-first part of a batch: every grid it holds beside one that it
+    does not, N - 2 at the edges of the matrix tiles (partial groups of tiles
+    included), then with one plan's lambda changed and one turned to Robin
+    faces (which leaves this path), against the oracle within twice its
+    rounding spread (or 1e-12)."""
+    from mpi_amd.solver import BatchSolver, HelmholtzPlan
+    sides, Ns = (32, 64, 128, 256), (130, 99, 67, 35, 98, 66, 34, 19, 33, 17, 9, 6, 18, 5, 4, 3)
+    specs = sorted(((nx, ny) for nx in sides for ny in sides), key=lambda s: s[0] * s[1])
+    specs = [(nx, ny, N) for (nx, ny), N in zip(specs, Ns)] + [(16, 64, 34), (32, 32, 3)]
+    geo = dict(xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2)
+    lam = [0.5 + i for i in range(len(specs))]
+    robin = [(0.0, 2.0, 0.0, -0.5)] * len(specs)
+    plans = [HelmholtzPlan(nx, ny, N, 1, lam=l, beta_l=2.0, beta_r=-0.5, form="diag", **geo)
+             for (nx, ny, N), l in zip(specs, lam)]
+    r = np.random.default_rng(7)
+    f = [r.standard_normal(s) for s in specs]
+    g = [[r.standard_normal(s[:2]) for s in specs] for _ in range(2)]
+    batch = BatchSolver(plans)
+    for rep in range(2):
+        us = batch.solve([to_dev(v) for v in f], [to_dev(v) for v in g[0]], [to_dev(v) for v in g[1]])
+        batch.status()
+        for k, (nx, ny, N) in enumerate(specs):
+            if rep and k not in (3, 5, 6):
+                continue
+            al, bl, ar, br = robin[k]
+            desc = po.make_desc(nx, ny, N, N, size=1, lam=lam[k], alphal=al, betal=bl, alphar=ar, betar=br, **geo)
+            uo, uf = (po.solve(desc, f[k], g[0][k], g[1][k], fma=m) for m in (False, True))
+            bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+            assert np.abs(us[k].cpu().numpy() - uo).max() <= bar * np.abs(uo).max(), (rep, specs[k])
+        lam[3], robin[5] = 40.0, (0.7, 1.3, 0.4, 2.0)
+        plans[3].set_lambda(lam[3])
+        plans[5].set_robin(*robin[5])
+    batch.close()
+    for p in plans:
+        p.close()
