@@ -138,10 +138,9 @@ struct ZfArgs {
     int nx, ny, K, n;
     int lr2;                    // log2(ny / 16)
     int ncol;                   // nx ny / 16 columns (x, n2)
-    const double *f;            // [nx][ny][K]: the right-hand side (adjoint: dL/du)
-    double *u;                  // [nx][ny][K]: the solution (adjoint: dL/df)
-    const double *gl, *gr;      // [nx][ny] (forward)
-    double *glbar, *grbar;      // [nx][ny] (adjoint)
+    const double *f;            // [nx][ny][K]: the right-hand side
+    double *u;                  // [nx][ny][K]: the solution
+    const double *gl, *gr;      // [nx][ny]
     double beta_l, beta_r;
     double *T;                  // [n][8][ncol] complex
     const double *B1, *B2;      // [NP][NP] contraction operands, row k, column j
@@ -151,12 +150,12 @@ struct ZfArgs {
     const double *mu;           // [n] eigenvalues, even ones first
     const double *sx, *sy;      // shifts lambda + kx^2 [nx/2 + 1], ky^2 [ny/2 + 1]
     const double2 *twx, *twy;
-    int adjoint, cubic;
+    int cubic;
     double c3, c1;              // cubic: the right-hand side f (c3 f^2 + c1)
 };
 bool zf_holds(int nx, int ny, int n);  // where one solve is faster this way
 int launch_zf(const ZfArgs &a, int stage, hipStream_t s);
-// The forward stages over many problems: every grid of zf_fits; work-group i
+// The stages over many problems: every grid of zf_fits; work-group i
 // takes tile list[i].y of problem Z[list[i].x], the entries of one launch being
 // of one zf_kind; a problem has zf_tasks tiles.
 bool zf_fits(int nx, int ny, int n);
@@ -299,9 +298,8 @@ struct hz_plan {
     double *d_eo_B1a = nullptr, *d_eo_B2a = nullptr;  // adjoint operands
     short *d_eo_M = nullptr, *d_eo_Ma = nullptr;      // first-order correction (bf16), forward and adjoint
     // z-first solve (zfirst.hip), where it applies (zf_route: and is faster for
-    // one solve alone): the operands in one
-    // allocation (forward B1, B2, X1, X2, then the adjoint's; w0, wN, mu), the
-    // bf16 corrections in another, and the shifts' two parts
+    // one solve alone): the operands in one allocation (B1, B2, X1, X2, w0, wN,
+    // mu), the bf16 corrections in another, and the shifts' two parts
     bool zf = false, zf_route = false;
     double *d_zf = nullptr, *d_zf_shift = nullptr;
     short *d_zf_C = nullptr;

@@ -251,7 +251,7 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
     static std::map<std::pair<std::vector<double>, int>, std::array<std::vector<short>, 2>> cache_m;
     static std::map<std::pair<std::vector<double>, int>, ZfOperands> cache_zf;
     // one element, Dirichlet faces, and a grid that the z-first kernels hold
-    const bool zf = zf_fits(p->nx, p->ny, n) && !diag_general(p);
+    const bool zf = p->d.form == HZ_FORM_DIAG && zf_fits(p->nx, p->ny, n) && !diag_general(p);
     ZfOperands zo;
     std::vector<double> mu, W, Wi;
     std::array<std::vector<short>, 2> Mq;
@@ -433,10 +433,9 @@ std::array<std::vector<short>, 2> correction_operator(const std::vector<long dou
 // and M: G_ij = M_ij / (mu_j - mu_i) between the halves, its entries outside
 // the first 16 x 16 block of each half rounded to bf16 as the kernels use
 // them, K = (I - G^2)^-1 (= I + G^2 + G^4 here: G^2 <= 1e-8).  With KW = K
-// Winv: forward B1 = KW^T, -G; B2 = (D W)^T, +G; adjoint B1 = D W, +G^T; B2 =
-// KW, -G^T; face loads K Winv F g: added before the correction (forward), or
-// against the corrected z (adjoint).  `d`: [B1, B2, X1, X2, w0, wN] forward, then
-// adjoint, then the n eigenvalues, even ones first; `c`: the four bf16 parts.
+// Winv: B1 = KW^T, -G; B2 = (D W)^T, +G; face loads K Winv F g, added before the
+// correction.  `d`: B1, B2, X1, X2 (G's FP64 block), w0, wN, then the n
+// eigenvalues, even ones first; `c`: the two bf16 parts.
 ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::vector<double> &W,
                        const std::vector<double> &Wi, const std::vector<long double> &M,
                        const std::vector<long double> &fg0, const std::vector<long double> &fgN)
@@ -448,8 +447,8 @@ ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::
     std::vector<double> G(Q, 0.0), G2(Q, 0.0), KW(Q, 0.0), K(Q, 0.0);
     ZfOperands o;
     const size_t set = 2 * Q + 1024 + 2 * NP;
-    o.d.assign(2 * set + n, 0.0);
-    o.c.assign(4 * Q, 0);
+    o.d.assign(set + n, 0.0);
+    o.c.assign(2 * Q, 0);
     for (int i = 0; i < NP; ++i)
         for (int j = 0; j < NP; ++j) {
             if (!real(i) || !real(j) || (i < H) == (j < H)) continue;
@@ -470,28 +469,22 @@ ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::
     product(K, G2, G2);
     KW = Wi;
     product(KW, K, Wi);  // (I + G^2 + G^4) Winv
-    double *f = o.d.data(), *ad = o.d.data() + set;
+    double *f = o.d.data();
     for (int k = 0; k < NP; ++k)
         for (int j = 0; j < NP; ++j) {
             auto dw = [&](int r, int c) { return (n % 2 && r == n / 2 ? 1.0 : 0.5) * W[(size_t)r * NP + c]; };
             f[(size_t)k * NP + j] = at(KW, j, k);
             f[Q + (size_t)k * NP + j] = dw(j, k);
-            ad[(size_t)k * NP + j] = dw(k, j);
-            ad[Q + (size_t)k * NP + j] = at(KW, k, j);
             if ((k < H) == (j < H)) continue;
-            const double g = at(G, j, k), gt = at(G, k, j);
+            const double g = at(G, j, k);
             if (k % H < 16 && j % H < 16) {
                 const size_t x = 2 * Q + (j < H ? 0 : 256) + (size_t)(k % H) * 16 + j % H;
                 f[x] = -g;
                 f[x + 512] = g;
-                ad[x] = gt;
-                ad[x + 512] = -gt;
             } else {
                 const size_t x = ((size_t)(k / 4) * NP + j) * 4 + k % 4;
                 o.c[x] = bf16_of(-g);
                 o.c[Q + x] = bf16_of(g);
-                o.c[2 * Q + x] = bf16_of(gt);
-                o.c[3 * Q + x] = bf16_of(-gt);
             }
         }
     const size_t vec = 2 * Q + 1024;
@@ -500,11 +493,10 @@ ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::
         std::vector<long double> w(NP, 0);
         for (int j = 0; j < NP; ++j)
             for (int k = 0; k < NP; ++k) w[j] += (long double)at(KW, j, k) * fg[k];
-        for (int j = 0; j < NP; ++j)
-            f[vec + (size_t)side * NP + j] = ad[vec + (size_t)side * NP + j] = real(j) ? (double)w[j] : 0.0;
+        for (int j = 0; j < NP; ++j) f[vec + (size_t)side * NP + j] = real(j) ? (double)w[j] : 0.0;
     }
-    for (int j = 0; j < he; ++j) o.d[2 * set + j] = mu[j];
-    for (int j = 0; j < ho; ++j) o.d[2 * set + he + j] = mu[H + j];
+    for (int j = 0; j < he; ++j) o.d[set + j] = mu[j];
+    for (int j = 0; j < ho; ++j) o.d[set + he + j] = mu[H + j];
     return o;
 }
 
@@ -574,11 +566,9 @@ int setup_diag(hz_plan *p)
 
 }  // namespace
 
-static ZfArgs zf_args_any(const hz_plan *p, bool adjoint, const double *f, double *u)
+ZfArgs hz::zf_args(const hz_plan *p, const double *f, double *u, const double *gl, const double *gr)
 {
-    const size_t Q = (size_t)p->NP * p->NP, set = 2 * Q + 1024 + 2 * p->NP;
-    const double *d = p->d_zf + (adjoint ? set : 0);
-    const short *c = p->d_zf_C + (adjoint ? 2 * Q : 0);
+    const size_t Q = (size_t)p->NP * p->NP;
     ZfArgs a{};
     a.nx = p->nx;
     a.ny = p->ny;
@@ -588,31 +578,24 @@ static ZfArgs zf_args_any(const hz_plan *p, bool adjoint, const double *f, doubl
     a.ncol = p->nx << a.lr2;
     a.f = f;
     a.u = u;
+    a.gl = gl;
+    a.gr = gr;
     a.beta_l = p->d.beta_l;
     a.beta_r = p->d.beta_r;
     a.T = p->spec.re;
-    a.B1 = d;
-    a.B2 = d + Q;
-    a.X1 = d + 2 * Q;
+    a.B1 = p->d_zf;
+    a.B2 = a.B1 + Q;
+    a.X1 = a.B2 + Q;
     a.X2 = a.X1 + 512;
     a.w0 = a.X2 + 512;
     a.wN = a.w0 + p->NP;
-    a.C1 = c;
-    a.C2 = c + Q;
-    a.mu = p->d_zf + 2 * set;
+    a.C1 = p->d_zf_C;
+    a.C2 = a.C1 + Q;
+    a.mu = a.wN + p->NP;
     a.sx = p->d_zf_shift;
     a.sy = p->d_zf_shift + p->nx / 2 + 1;
     a.twx = p->d_twx;
     a.twy = p->d_twy;
-    a.adjoint = adjoint;
-    return a;
-}
-
-ZfArgs hz::zf_args(const hz_plan *p, const double *f, double *u, const double *gl, const double *gr)
-{
-    ZfArgs a = zf_args_any(p, false, f, u);
-    a.gl = gl;
-    a.gr = gr;
     return a;
 }
 
@@ -1224,17 +1207,12 @@ int hz_plan_set_robin(hz_plan *p, double alpha_l, double beta_l, double alpha_r,
     return HZ_OK;
 }
 
-// The one-element Dirichlet solve or its adjoint (f = dL/du, u = dL/df) with
-// the z contractions outside the transforms (zfirst.hip); the plan's spectrum
-// is the intermediate.
-static int zf_pipeline(hz_plan *p, const double *f, double *u, const double *gl, const double *gr, double *glbar,
-                       double *grbar, const double *cubic, hipStream_t s, StageRecorder *rec)
+// The one-element Dirichlet solve with the z contractions outside the
+// transforms (zfirst.hip); the plan's spectrum is the intermediate.
+static int zf_pipeline(hz_plan *p, const double *f, double *u, const double *gl, const double *gr,
+                       const double *cubic, hipStream_t s, StageRecorder *rec)
 {
-    ZfArgs a = zf_args_any(p, glbar != nullptr, f, u);
-    a.gl = gl;
-    a.gr = gr;
-    a.glbar = glbar;
-    a.grbar = grbar;
+    ZfArgs a = zf_args(p, f, u, gl, gr);
     if (cubic) {
         a.cubic = 1;
         a.c3 = cubic[0];
@@ -1260,7 +1238,7 @@ static int solve_impl(hz_plan *p, const double *f, const double *gl, const doubl
     }
     StageRecorder rec(p, s);
     if (p->d.form == HZ_FORM_DIAG && p->zf_route && !diag_general(p) && !op_diag && !op_full)
-        return zf_pipeline(p, f, u, gl, gr, nullptr, nullptr, cubic, s, &rec);
+        return zf_pipeline(p, f, u, gl, gr, cubic, s, &rec);
     int st = forward_xy(p, f, p->spec.re, p->spec.im, p->K, s, gl, gr, p->xs, cubic);
     rec.mark("fft_forward");
     if (st) return st;
@@ -1374,7 +1352,6 @@ static int adjoint_pipeline(hz_plan *p, const double *ubar, double *fbar, double
                             hipStream_t s, StageRecorder *rec)
 {
     int st;
-    if (p->zf_route && !diag_general(p)) return zf_pipeline(p, ubar, fbar, nullptr, nullptr, glbar, grbar, nullptr, s, rec);
     if ((st = forward_xy(p, ubar, p->spec.re, p->spec.im, p->K, s, nullptr, nullptr, p->xs))) return st;
     if (rec) rec->mark("fft_forward");
     DiagArgs a = diag_args(p);
@@ -1425,7 +1402,7 @@ int hz_adjoint(hz_plan *p, const double *ubar, const double *u, double *fbar, do
     if ((st = adjoint_args(p, ubar, u, fbar, glbar, grbar, lambda_bar))) return st;
     const hipStream_t s = (hipStream_t)stream;
     if (!p->d_Vrow) {
-        if ((st = setup_diag(p)) || (st = compute_homogeneous(p)) || (st = zf_shifts(p))) return st;
+        if ((st = setup_diag(p)) || (st = compute_homogeneous(p))) return st;
     }
     StageRecorder rec(p, s);
     if ((st = adjoint_pipeline(p, ubar, fbar, glbar, grbar, s, &rec))) return st;

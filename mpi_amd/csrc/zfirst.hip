@@ -1,4 +1,4 @@
-// zfirst.hip -- the one-element Dirichlet solve (and its adjoint) with the z
+// zfirst.hip -- the one-element Dirichlet solve with the z
 // contractions outside the x-y transforms, in three kernels.
 //
 // With the even/odd eigenbasis of the interior operator (diag_body.h) the
@@ -17,8 +17,11 @@
 //                 end values, the store of u.
 // Against transform - mode solve - transform this is three reads and writes
 // of the field instead of five and no transform of the face data (Dirichlet
-// values are added and returned in physical space): 165 -> 132 us a solve and
-// 180 -> 134 us an adjoint at 256^2 x 130.
+// values are added and returned in physical space): 165 -> 135 us a solve at
+// 256^2 x 130.  The adjoint stays with transform - mode solve - transform: its
+// sum against the solution, dL/dlambda, cancels to a millionth of its terms, and
+// the contractions' rounding, which reaches the quiet (kx, ky) here, left that
+// sum up to ten times as far off.
 //
 // With ny = 16 R2, y = n2 + R2 n1 and ky = k1 + 16 k2: kernel 1 owns 4
 // columns (x, n2) and all 16 n1 of each.  Rows are dealt to the matrix tiles
@@ -35,7 +38,7 @@
 // (I - G) K V^-1 with K = (I - G^2)^-1 (block diagonal, folded into the
 // operand).  The largest eigenvalues come in nearly equal even/odd pairs, so
 // G reaches 1e-6 there (N = 130): its first 16 x 16 block runs in FP64, the
-// rest (below 3e-11) with bf16 operands and FP32 sums.
+// rest (below 3e-11) in bf16 with FP32 sums, the values in two parts.
 #include "diag_body.h"
 #include "fft_body.h"
 
@@ -176,19 +179,23 @@ struct RowAt {
     }
 };
 
-// The correction's operands in the LDS of the tile: the values in bf16 (row
-// stride LDB shorts: 16 rows x 4 lane groups of 8 bytes spread over the banks)
-// and the first 16 of each half in FP64 (row stride 34).  Each wave rounds its
-// own values once; 48 KB less LDS is read than when every wave takes the FP64
-// tile and rounds what it reads.
+// The correction's operands in the LDS of the tile: every value as two bf16
+// parts, its rounding and the rounding of the rest (groups of four values: four
+// first parts, four second ones; 16 rows x 4 lane groups of 16 bytes spread over
+// the banks), and the first 16 of each half in FP64 (row stride 34).  The two
+// corrections nearly cancel in the solution, their roundings do not: with one
+// part the sum of fbar u was three times as far off.  At NP = 32 the FP64 block
+// is all of G.
 template <int NJ>
 struct CorrLds {
-    static constexpr int LDB = 16 * NJ + 4, LDX = 34;
-    static constexpr int XOFF = kRows * LDB / 4;  // doubles
-    static_assert(XOFF + kRows * LDX <= kRows * (16 * NJ + 2) || NJ < 4, "inside the tile");
+    static constexpr int LDB = 32 * NJ + 8, LDX = 34;
+    static constexpr int XOFF = NJ > 2 ? kRows * LDB / 4 : 0;  // doubles
     static constexpr int DOUBLES = XOFF + kRows * LDX > kRows * (16 * NJ + 2) ? XOFF + kRows * LDX
                                                                               : kRows * (16 * NJ + 2);
 };
+
+typedef short s8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 // LDS of one tile of an end kernel.
 template <int NJ>
@@ -201,12 +208,19 @@ template <int NJ>
 __device__ __forceinline__ void to_corr(const d4 (&acc)[4][1], double *tile, int w, int li, int lk)
 {
     using S = CorrLds<NJ>;
-    __bf16 *tb = reinterpret_cast<__bf16 *>(tile);
-    const int j = 16 * w + li;
+    if constexpr (NJ > 2) {
+        __bf16 *tb = reinterpret_cast<__bf16 *>(tile) + 8 * ((16 * w + li) / 4) + li % 4;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+        for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tb[(16 * rb + 4 * r + lk) * S::LDB + j] = (__bf16)(float)acc[rb][0][r];
+            for (int r = 0; r < 4; ++r) {
+                const float v = (float)acc[rb][0][r];
+                const __bf16 hi = (__bf16)v;
+                __bf16 *t = tb + (16 * rb + 4 * r + lk) * S::LDB;
+                t[0] = hi;
+                t[4] = (__bf16)(v - (float)hi);
+            }
+    }
     if (w % (NJ / 2) == 0) {
         double *tx = tile + S::XOFF + (w ? 16 : 0) + li;
 #pragma unroll
@@ -229,23 +243,68 @@ __device__ __forceinline__ void correct(d4 (&acc)[4][1], const double *tile, con
     f4 cacc[4];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) cacc[rb] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const s4 *bq = reinterpret_cast<const s4 *>(C) + (ko / 4 + lk) * NP + 16 * w + li;
-    const short *arow = reinterpret_cast<const short *>(tile) + (4 * (li % 4) + li / 4) * S::LDB + ko + 4 * lk;
+    if constexpr (NJ > 2) {
+        // one 16x16x32 step: 16 values, their two parts against the same operand
+        const s4 *bq = reinterpret_cast<const s4 *>(C) + (ko / 4 + lk) * NP + 16 * w + li;
+        const short *arow = reinterpret_cast<const short *>(tile) + (4 * (li % 4) + li / 4) * S::LDB + 2 * ko + 8 * lk;
 #pragma unroll
-    for (int ks = 0; ks < H / 16; ++ks) {
-        const s4 bv = bq[4 * ks * NP];
+        for (int ks = 0; ks < H / 16; ++ks) {
+            const s4 b = bq[4 * ks * NP];
+            const s8 bv = {b[0], b[1], b[2], b[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            const s4 av = *reinterpret_cast<const s4 *>(arow + 16 * rb * S::LDB + 16 * ks);
-            cacc[rb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, cacc[rb], 0, 0, 0);
+            for (int rb = 0; rb < 4; ++rb) {
+                const s8 av = *reinterpret_cast<const s8 *>(arow + 16 * rb * S::LDB + 32 * ks);
+                cacc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, av),
+                                                                   __builtin_bit_cast(bf8, bv), cacc[rb], 0, 0, 0);
+            }
         }
     }
     if (w % (NJ / 2) == 0)  // the first 16 of each half
         tile_gemm_deep<16, S::LDX, 4, 1, 16, 4>(acc, tile + S::XOFF + (w ? 0 : 16), X + (w ? 256 : 0), 0, 0, li, lk);
+    if constexpr (NJ > 2) {
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+        for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[rb][0][r] += (double)cacc[rb][r];
+            for (int r = 0; r < 4; ++r) acc[rb][0][r] += (double)cacc[rb][r];
+    }
+}
+
+// acc = A B over the wave's half (operands as pair_gemm), each half of the sum
+// on its own.  Here the contractions run in physical space, where their
+// rounding reaches every (kx, ky), also the quiet ones, and a sum's rounding
+// grows with its partial sums: two shorter ones halve it.
+template <int NJ>
+__device__ __forceinline__ void contract(d4 (&acc)[4][1], const double *tile, const double *__restrict__ B, int j,
+                                         int li, int lk)
+{
+    constexpr int NP = 16 * NJ, LD = NP + 2, NPR = NP / 16, D = 2;
+    const double *bc = B + 2 * lk * NP + j;
+    d4 sum[2][4];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) sum[0][rb] = sum[1][rb] = d4{0.0, 0.0, 0.0, 0.0};
+    double b[D][2];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        b[d][0] = bc[8 * d * NP];
+        b[d][1] = bc[(8 * d + 1) * NP];
+    }
+#pragma unroll
+    for (int p = 0; p < NPR; ++p) {
+        const double v0 = b[p % D][0], v1 = b[p % D][1];
+        if (p + D < NPR) {
+            b[p % D][0] = bc[8 * (p + D) * NP];
+            b[p % D][1] = bc[(8 * (p + D) + 1) * NP];
+        }
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+            const double2 av = *reinterpret_cast<const double2 *>(tile + (16 * rb + li) * LD + 8 * p + 2 * lk);
+            d4 &c = sum[2 * p / NPR][rb];
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, v0, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, v1, c, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) acc[rb][0] = sum[0][rb] + sum[1][rb];
 }
 
 template <int NJ>
@@ -272,20 +331,18 @@ __device__ __forceinline__ int compact(int j, int he, int ho)
 // work-group's life), contraction (24%, near the matrix rate of the two that
 // share a CU), correction (20%) and stores hardly overlap: without the loads
 // 41 us, without the contraction 33, without the stores 44.
-template <int NJ, bool ADJ, bool CUB>
+template <int NJ, bool CUB>
 __device__ __forceinline__ void expand_tile(const ZfArgs &a, int c0, int tid, EndLds<NJ> &lds)
 {
     constexpr int NP = 16 * NJ, LD = NP + 2, H = NP / 2, T = 64 * NJ;
     double *tile = lds.tile, *row_zl = lds.rows[0], *row_zr = lds.rows[1];
     const int lane = tid % 64, w = uniform(tid / 64), li = lane % 16, lk = lane / 16;
     const int n = a.n, ho = n / 2, he = n - ho;
-    if constexpr (!ADJ) {
-        if (tid < kRows) {
-            const RowAt at(tid, c0, a.lr2);
-            const int g = at.x * a.ny + at.y;
-            row_zl[tid] = a.gl[g] / a.beta_l;
-            row_zr[tid] = a.gr[g] / a.beta_r;
-        }
+    if (tid < kRows) {
+        const RowAt at(tid, c0, a.lr2);
+        const int g = at.x * a.ny + at.y;
+        row_zl[tid] = a.gl[g] / a.beta_l;
+        row_zr[tid] = a.gr[g] / a.beta_r;
     }
     {
         // folded interior: even coordinate i f_i + f_(n-1-i) (the centre of an
@@ -313,19 +370,15 @@ __device__ __forceinline__ void expand_tile(const ZfArgs &a, int c0, int tid, En
     __syncthreads();
     const int kb = 16 * w >= H ? H : 0;  // the wave's half
     d4 acc[4][1];
+    contract<NJ>(acc, tile + kb, a.B1 + kb * NP, 16 * w + li, li, lk);
+    const double w0 = a.w0[16 * w + li], wN = a.wN[16 * w + li];
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) acc[rb][0] = d4{0.0, 0.0, 0.0, 0.0};
-    tile_gemm_deep<NP, LD, 4, 1, H, 4>(acc, tile + kb, a.B1 + (long long)kb * NP, w, 0, li, lk);
-    if constexpr (!ADJ) {
-        const double w0 = a.w0[16 * w + li], wN = a.wN[16 * w + li];
+    for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * rb + 4 * r + lk;
-                acc[rb][0][r] += fma(row_zl[row], w0, row_zr[row] * wN);
-            }
-    }
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * rb + 4 * r + lk;
+            acc[rb][0][r] += fma(row_zl[row], w0, row_zr[row] * wN);
+        }
     __syncthreads();  // every wave has read the folded tile
     to_corr<NJ>(acc, tile, w, li, lk);
     __syncthreads();
@@ -342,13 +395,12 @@ __device__ __forceinline__ void expand_tile(const ZfArgs &a, int c0, int tid, En
 }
 
 // ---- 3: 16-point stage back, correction, contraction, store --------------------
-// zf_expand's mirror image and bounds; 256^2 x 129: 55 us (adjoint 57).
-template <int NJ, bool ADJ>
+// zf_expand's mirror image and bounds; 256^2 x 129: 56 us.
+template <int NJ>
 __device__ __forceinline__ void collect_tile(const ZfArgs &a, int c0, int tid, EndLds<NJ> &lds)
 {
     constexpr int NP = 16 * NJ, LD = NP + 2, H = NP / 2, T = 64 * NJ;
     double *tile = lds.tile;
-    auto &face = lds.rows;
     const int lane = tid % 64, w = uniform(tid / 64), li = lane % 16, lk = lane / 16;
     const int n = a.n, ho = n / 2, he = n - ho;
     const int jc = compact<H>(16 * w + li, he, ho);
@@ -374,48 +426,13 @@ __device__ __forceinline__ void collect_tile(const ZfArgs &a, int c0, int tid, E
     __syncthreads();  // every wave has read the uncorrected values
     to_tile<NJ>(acc, tile, w, li, lk);
     __syncthreads();
-    if constexpr (ADJ) {
-        // face gradients: w0|wN . z of every row, NJ threads a row (w0, wN in
-        // the basis of the corrected z)
-        const int row = tid / NJ, part = tid % NJ;
-        double s0 = 0.0, sN = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const double z = tile[row * LD + part + NJ * k];
-            s0 = fma(a.w0[part + NJ * k], z, s0);
-            sN = fma(a.wN[part + NJ * k], z, sN);
-        }
-#pragma unroll
-        for (int o = 1; o < (NJ == 6 ? 2 : NJ); o <<= 1) {
-            s0 += __shfl_xor(s0, o);
-            sN += __shfl_xor(sN, o);
-        }
-        if constexpr (NJ == 6) {  // three pairs
-            // a row's 6 threads may straddle two waves: through LDS
-            __shared__ double pairs[2][kRows][3];
-            if (part % 2 == 0) {
-                pairs[0][row][part / 2] = s0;
-                pairs[1][row][part / 2] = sN;
-            }
-            __syncthreads();
-            if (part == 0) {
-                face[0][row] = (pairs[0][row][0] + pairs[0][row][1]) + pairs[0][row][2];
-                face[1][row] = (pairs[1][row][0] + pairs[1][row][1]) + pairs[1][row][2];
-            }
-        } else if (part == 0) {
-            face[0][row] = s0;
-            face[1][row] = sN;
-        }
-    }
     const int kb = 16 * w >= H ? H : 0;
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) acc[rb][0] = d4{0.0, 0.0, 0.0, 0.0};
-    tile_gemm_deep<NP, LD, 4, 1, H, 4>(acc, tile + kb, a.B2 + (long long)kb * NP, w, 0, li, lk);
+    contract<NJ>(acc, tile + kb, a.B2 + kb * NP, 16 * w + li, li, lk);
     __syncthreads();
     to_tile<NJ>(acc, tile, w, li, lk);
     __syncthreads();
     // u_i = e_i + o_i, u_(n-1-i) = e_i - o_i, the centre of an odd n e_i; the
-    // end values are the faces' (the adjoint load has none)
+    // end values are the faces'
     for (int idx = tid; idx < kRows * NP; idx += T) {
         const int row = idx / NP, k = idx % NP;
         if (k >= n) continue;
@@ -429,28 +446,22 @@ __device__ __forceinline__ void collect_tile(const ZfArgs &a, int c0, int tid, E
         const int row = tid >> 1, side = tid & 1;
         const RowAt at(row, c0, a.lr2);
         const int g = at.x * a.ny + at.y, end = g * a.K + (side ? n + 1 : 0);
-        if constexpr (ADJ) {
-            const double v = (a.f[end] + face[side][row]) / (side ? a.beta_r : a.beta_l);
-            (side ? a.grbar : a.glbar)[g] = v;
-            a.u[end] = 0.0;
-        } else {
-            a.u[end] = side ? a.gr[g] / a.beta_r : a.gl[g] / a.beta_l;
-        }
+        a.u[end] = side ? a.gr[g] / a.beta_r : a.gl[g] / a.beta_l;
     }
 }
 
-template <int NJ, bool ADJ, bool CUB>
+template <int NJ, bool CUB>
 __global__ __launch_bounds__(64 * NJ, 4) void zf_expand(const ZfArgs a)
 {
     __shared__ EndLds<NJ> lds;
-    expand_tile<NJ, ADJ, CUB>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
+    expand_tile<NJ, CUB>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
 }
 
-template <int NJ, bool ADJ>
+template <int NJ>
 __global__ __launch_bounds__(64 * NJ, NJ == 6 ? 3 : 4) void zf_collect(const ZfArgs a)
 {
     __shared__ EndLds<NJ> lds;
-    collect_tile<NJ, ADJ>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
+    collect_tile<NJ>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
 }
 
 // Many problems: one (problem, tile) entry per work-group.  Pointers read from
@@ -504,9 +515,9 @@ __device__ __forceinline__ void end_tiles_of(const ZfArgs &a, int task, char *sm
     if (sub >= PER || 4 * t >= a.ncol) return;  // waves that ended take no part in the barriers
     EndLds<NJ> &lds = reinterpret_cast<EndLds<NJ> *>(smem)[sub];
     if constexpr (COLLECT)
-        collect_tile<NJ, false>(a, 4 * t, threadIdx.x % T, lds);
+        collect_tile<NJ>(a, 4 * t, threadIdx.x % T, lds);
     else
-        expand_tile<NJ, false, false>(a, 4 * t, threadIdx.x % T, lds);
+        expand_tile<NJ, false>(a, 4 * t, threadIdx.x % T, lds);
 }
 
 // Every problem of a batch in one launch: its tasks of different sizes fill the
@@ -517,7 +528,7 @@ template <bool COLLECT>
 __global__ __launch_bounds__(512, 4) void zf_end_list(const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
 {
     __shared__ alignas(16) char smem[2 * sizeof(EndLds<4>)];
-    static_assert(sizeof(smem) >= sizeof(EndLds<8>) && sizeof(smem) >= 3 * sizeof(EndLds<2>), "every size fits");
+    static_assert(sizeof(smem) >= sizeof(EndLds<8>) && sizeof(smem) >= end_tiles(2) * sizeof(EndLds<2>), "every size fits");
     const int2 e = list[xcd_logical(blockIdx.x, gridDim.x)];
     const ZfArgs a = problem_args(Z, uniform(e.x));
     const int task = uniform(e.y);
@@ -759,18 +770,12 @@ template <int NJ>
 int launch_ends(const ZfArgs &a, bool collect, hipStream_t s)
 {
     const dim3 grid(a.ncol / 4), block(64 * NJ);
-    if (collect) {
-        if (a.adjoint)
-            hipLaunchKernelGGL((zf_collect<NJ, true>), grid, block, 0, s, a);
-        else
-            hipLaunchKernelGGL((zf_collect<NJ, false>), grid, block, 0, s, a);
-    } else if (a.adjoint) {
-        hipLaunchKernelGGL((zf_expand<NJ, true, false>), grid, block, 0, s, a);
-    } else if (a.cubic) {
-        hipLaunchKernelGGL((zf_expand<NJ, false, true>), grid, block, 0, s, a);
-    } else {
-        hipLaunchKernelGGL((zf_expand<NJ, false, false>), grid, block, 0, s, a);
-    }
+    if (collect)
+        hipLaunchKernelGGL(zf_collect<NJ>, grid, block, 0, s, a);
+    else if (a.cubic)
+        hipLaunchKernelGGL((zf_expand<NJ, true>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((zf_expand<NJ, false>), grid, block, 0, s, a);
     HZ_HIP(hipGetLastError());
     return HZ_OK;
 }
