@@ -87,7 +87,7 @@ __device__ __forceinline__ void coop_mixed_t(const MixedArgs &a, int t, double *
 }
 
 // A mode-solve task: tile t of the problem's DIAG (kind 0-7) or MIXED
-// (kind 8-15, the tile heights of mixed_tile_rows) kernel body.
+// (kind 8-15) kernel body.
 template <int RT>
 __device__ __noinline__ void coop_modes(const BatchProblem &pr, int t, double *smem)
 {
@@ -102,12 +102,12 @@ __device__ __noinline__ void coop_modes(const BatchProblem &pr, int t, double *s
     case 7: coop_diag_t<8, RT, true>(pr.d, t, smem); break;
     case 8: coop_mixed_t<2, 32, false>(pr.m, t, smem); break;
     case 9: coop_mixed_t<2, 32, true>(pr.m, t, smem); break;
-    case 10: coop_mixed_t<4, 16, false>(pr.m, t, smem); break;
-    case 11: coop_mixed_t<4, 16, true>(pr.m, t, smem); break;
+    case 10: coop_mixed_t<4, 32, false>(pr.m, t, smem); break;
+    case 11: coop_mixed_t<4, 32, true>(pr.m, t, smem); break;
     case 12: coop_mixed_t<6, 32, false>(pr.m, t, smem); break;
     case 13: coop_mixed_t<6, 32, true>(pr.m, t, smem); break;
-    case 14: coop_mixed_t<8, 16, false>(pr.m, t, smem); break;
-    default: coop_mixed_t<8, 16, true>(pr.m, t, smem); break;
+    case 14: coop_mixed_t<8, 32, false>(pr.m, t, smem); break;
+    default: coop_mixed_t<8, 32, true>(pr.m, t, smem); break;
     }
 }
 
@@ -138,9 +138,9 @@ constexpr size_t coop_lds()
     m = cmax(m, sizeof(DiagShared<6, RT, true, false>));
     m = cmax(m, sizeof(DiagShared<8, RT, true, false>));
     m = cmax(m, sizeof(MixedShared<2, 32, true>));
-    m = cmax(m, sizeof(MixedShared<4, 16, true>));
+    m = cmax(m, sizeof(MixedShared<4, 32, true>));
     m = cmax(m, sizeof(MixedShared<6, 32, true>));
-    m = cmax(m, sizeof(MixedShared<8, 16, true>));
+    m = cmax(m, sizeof(MixedShared<8, 32, true>));
     return m;
 }
 
@@ -252,12 +252,12 @@ __global__ __launch_bounds__(256) void batch_stage_modes(const BatchProblem *__r
     case 7: coop_diag_t<8, RT, true>(pr.d, e.y, smem); break;
     case 8: coop_mixed_t<2, 32, false>(pr.m, e.y, smem); break;
     case 9: coop_mixed_t<2, 32, true>(pr.m, e.y, smem); break;
-    case 10: coop_mixed_t<4, 16, false>(pr.m, e.y, smem); break;
-    case 11: coop_mixed_t<4, 16, true>(pr.m, e.y, smem); break;
+    case 10: coop_mixed_t<4, 32, false>(pr.m, e.y, smem); break;
+    case 11: coop_mixed_t<4, 32, true>(pr.m, e.y, smem); break;
     case 12: coop_mixed_t<6, 32, false>(pr.m, e.y, smem); break;
     case 13: coop_mixed_t<6, 32, true>(pr.m, e.y, smem); break;
-    case 14: coop_mixed_t<8, 16, false>(pr.m, e.y, smem); break;
-    default: coop_mixed_t<8, 16, true>(pr.m, e.y, smem); break;
+    case 14: coop_mixed_t<8, 32, false>(pr.m, e.y, smem); break;
+    default: coop_mixed_t<8, 32, true>(pr.m, e.y, smem); break;
     }
 }
 
@@ -296,6 +296,26 @@ __global__ __launch_bounds__(256) void batch_unit_list(const BatchProblem *__res
     unit_line_element<KIND>(P[t.x].f[pass], (long long)t.y * 256 + threadIdx.x);
 }
 
+__device__ __forceinline__ MixedArgs global_args(MixedArgs a)
+{
+    a.spec = as_global(a.spec);
+    a.bc_re = as_global(a.bc_re);
+    a.bc_im = as_global(a.bc_im);
+    a.shift = as_global(a.shift);
+    a.mu = as_global(a.mu);
+    a.VinvT32 = as_global(a.VinvT32);
+    a.VT32 = as_global(a.VT32);
+    a.DzzTP = as_global(a.DzzTP);
+    a.Dzz = as_global(a.Dzz);
+    a.Dz = as_global(a.Dz);
+    a.UL = as_global(a.UL);
+    a.UR = as_global(a.UR);
+    a.hom = as_global(a.hom);
+    a.hist = as_global(a.hist);
+    a.closure = as_global(a.closure);
+    return a;
+}
+
 template <int NJ, int RT, bool GENERAL>
 __global__ __launch_bounds__(256) void batch_diag_list(const BatchProblem *__restrict__ P, const int2 *__restrict__ list)
 {
@@ -304,13 +324,14 @@ __global__ __launch_bounds__(256) void batch_diag_list(const BatchProblem *__res
     diag_tile<NJ, RT, GENERAL, false>(P[t.x].d, t.y, sh);
 }
 
-template <int NJ, int RT, bool GENERAL>
-__global__ __launch_bounds__(256, 2) void batch_mixed_list(const BatchProblem *__restrict__ P,
-                                                           const int2 *__restrict__ list)
+// One wave per 16 columns (mixed_waves_tile), 32 rows: 48 problems of 32 to 128
+// points a side 640 us, with mixed_tile's four waves a tile 877.
+template <int NJ, bool GENERAL>
+__global__ __launch_bounds__(64 * NJ, NJ == 6 && GENERAL ? 3 : 4) void batch_mixed_list(
+    const BatchProblem *__restrict__ P, const int2 *__restrict__ list)
 {
-    __shared__ MixedShared<NJ, RT, GENERAL> sh;
     const int2 t = list[blockIdx.x];
-    mixed_tile<NJ, RT, GENERAL>(P[t.x].m, t.y, sh);
+    mixed_waves_tile<NJ, 2, GENERAL>(global_args(P[uniform(t.x)].m), uniform(t.y));
 }
 
 }  // namespace
@@ -391,10 +412,10 @@ namespace {
 int rt_index(int rt) { return rt == 64 ? 1 : 0; }
 
 // Mode-solve tiles of a plan for DIAG tiles of `rt` rows (MIXED tiles have
-// a fixed height per padded size).
+// 32).
 int mode_tiles(const hz_plan *pl, int rt)
 {
-    const int rows = pl->d.form == HZ_FORM_MIXED ? mixed_tile_rows(diag_padded(pl->n)) : rt;
+    const int rows = pl->d.form == HZ_FORM_MIXED ? 32 : rt;
     const int fc_per_tile = rows / (2 * pl->ne);
     const int nfc = pl->nx * pl->M;
     return (nfc + fc_per_tile - 1) / fc_per_tile;
@@ -450,16 +471,16 @@ void launch_fft_list(hipStream_t s, const BatchProblem *P, const int2 *list, int
 
 void launch_mixed_list(hipStream_t s, const BatchProblem *P, const int2 *list, int count, int kind)
 {
-    const dim3 g(count), b(256);
-    switch (kind) {  // MIXED tile heights: mixed_tile_rows
-    case 0: hipLaunchKernelGGL((batch_mixed_list<2, 32, false>), g, b, 0, s, P, list); break;
-    case 1: hipLaunchKernelGGL((batch_mixed_list<2, 32, true>), g, b, 0, s, P, list); break;
-    case 2: hipLaunchKernelGGL((batch_mixed_list<4, 16, false>), g, b, 0, s, P, list); break;
-    case 3: hipLaunchKernelGGL((batch_mixed_list<4, 16, true>), g, b, 0, s, P, list); break;
-    case 4: hipLaunchKernelGGL((batch_mixed_list<6, 32, false>), g, b, 0, s, P, list); break;
-    case 5: hipLaunchKernelGGL((batch_mixed_list<6, 32, true>), g, b, 0, s, P, list); break;
-    case 6: hipLaunchKernelGGL((batch_mixed_list<8, 16, false>), g, b, 0, s, P, list); break;
-    default: hipLaunchKernelGGL((batch_mixed_list<8, 16, true>), g, b, 0, s, P, list); break;
+    const dim3 g(count), b(128 * (kind / 2 + 1));
+    switch (kind) {
+    case 0: hipLaunchKernelGGL((batch_mixed_list<2, false>), g, b, 0, s, P, list); break;
+    case 1: hipLaunchKernelGGL((batch_mixed_list<2, true>), g, b, 0, s, P, list); break;
+    case 2: hipLaunchKernelGGL((batch_mixed_list<4, false>), g, b, 0, s, P, list); break;
+    case 3: hipLaunchKernelGGL((batch_mixed_list<4, true>), g, b, 0, s, P, list); break;
+    case 4: hipLaunchKernelGGL((batch_mixed_list<6, false>), g, b, 0, s, P, list); break;
+    case 5: hipLaunchKernelGGL((batch_mixed_list<6, true>), g, b, 0, s, P, list); break;
+    case 6: hipLaunchKernelGGL((batch_mixed_list<8, false>), g, b, 0, s, P, list); break;
+    default: hipLaunchKernelGGL((batch_mixed_list<8, true>), g, b, 0, s, P, list); break;
     }
 }
 

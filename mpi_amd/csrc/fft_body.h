@@ -54,6 +54,15 @@ __device__ __forceinline__ T sval(T v)
     return (T)(((unsigned long long)hi << 32) | lo);
 }
 
+// A wave-uniform pointer that was read from memory, marked as a global one (as
+// pointers among kernel arguments are): generic loads and stores would wait on
+// the LDS counter as well.
+template <class V>
+__device__ __forceinline__ V *as_global(V *p)
+{
+    return (V *)(V __attribute__((address_space(1))) *)sval((unsigned long long)p);
+}
+
 // In-register R-point DFT, radix-2 decimation in time.  tw holds the
 // L-point table; W_R^t = tw[t * (L/R)].  SIGN = -1 forward, +1 inverse.
 template <int R, int L, int SIGN>

@@ -464,14 +464,8 @@ __global__ __launch_bounds__(64 * NJ, NJ == 6 ? 3 : 4) void zf_collect(const ZfA
     collect_tile<NJ>(a, 4 * xcd_logical(blockIdx.x, gridDim.x), threadIdx.x, lds);
 }
 
-// Many problems: one (problem, tile) entry per work-group.  Pointers read from
-// memory are marked as global ones (as kernel arguments are): generic loads
-// would wait on the LDS counter as well and cost the filter 100 registers.
-template <class V>
-__device__ __forceinline__ V *as_global(V *p)
-{
-    return (V *)(V __attribute__((address_space(1))) *)sval((unsigned long long)p);
-}
+// Many problems: one (problem, tile) entry per work-group (generic loads would
+// cost the filter 100 registers).
 __device__ __forceinline__ ZfArgs problem_args(const ZfArgs *__restrict__ Z, int p)
 {
     ZfArgs a = Z[p];
