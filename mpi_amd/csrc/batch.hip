@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256) void batch_diag_list(const BatchProblem *__res
 }
 
 // One wave per 16 columns (mixed_waves_tile), 32 rows: 48 problems of 32 to 128
-// points a side 640 us, with mixed_tile's four waves a tile 877.
+// points a side 618 us, with mixed_tile's four waves a tile 877.
 template <int NJ, bool GENERAL>
 __global__ __launch_bounds__(64 * NJ, NJ == 6 && GENERAL ? 3 : 4) void batch_mixed_list(
     const BatchProblem *__restrict__ P, const int2 *__restrict__ list)

@@ -434,7 +434,7 @@ __device__ __forceinline__ void mixed_waves_tile(const MixedArgs &a, int bx)
 {
     constexpr int NP = 16 * NJ, H = NP / 2, RT = 16 * RB, T = 64 * NJ, KS = H / 4;
     constexpr int LD = NP + 2, LDF = NP + 4;   // conflict-free row strides
-    // separate arrays: as fields of one, they cost the kernel 84 bytes of spills (202 -> 225 us)
+    // separate arrays: as fields of one they cost 84 bytes of spills (a 256^2 x 129 solve 293 -> 317 us)
     __shared__ alignas(16) double x[RT * LD];  // the iterate
     __shared__ alignas(16) float t[RT * LDF];  // FP32 right-hand sides, then the folded solution
     __shared__ alignas(16) float z[RT * LDF];  // scaled eigen coordinates

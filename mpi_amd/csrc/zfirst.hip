@@ -522,7 +522,8 @@ template <bool COLLECT>
 __global__ __launch_bounds__(512, 4) void zf_end_list(const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
 {
     __shared__ alignas(16) char smem[2 * sizeof(EndLds<4>)];
-    static_assert(sizeof(smem) >= sizeof(EndLds<8>) && sizeof(smem) >= end_tiles(2) * sizeof(EndLds<2>), "every size fits");
+    static_assert(sizeof(smem) >= sizeof(EndLds<8>) && sizeof(smem) >= end_tiles(2) * sizeof(EndLds<2>),
+                  "every size fits");
     const int2 e = list[xcd_logical(blockIdx.x, gridDim.x)];
     const ZfArgs a = problem_args(Z, uniform(e.x));
     const int task = uniform(e.y);
