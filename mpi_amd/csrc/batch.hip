@@ -80,14 +80,8 @@ __device__ __forceinline__ void coop_diag_t(const DiagArgs &a, int t, double *sm
     diag_tile<NJ, RT, GENERAL, false>(a, t, *reinterpret_cast<DiagShared<NJ, RT, GENERAL, false> *>(smem));
 }
 
-template <int NJ, int RT, bool GENERAL>
-__device__ __forceinline__ void coop_mixed_t(const MixedArgs &a, int t, double *smem)
-{
-    mixed_tile<NJ, RT, GENERAL>(a, t, *reinterpret_cast<MixedShared<NJ, RT, GENERAL> *>(smem));
-}
-
-// A mode-solve task: tile t of the problem's DIAG (kind 0-7) or MIXED
-// (kind 8-15) kernel body.
+// A mode-solve task: tile t of the problem's DIAG kernel body (kinds 0-7; a
+// batch with other kinds is not run fused, see variant_usable).
 template <int RT>
 __device__ __noinline__ void coop_modes(const BatchProblem &pr, int t, double *smem)
 {
@@ -99,15 +93,7 @@ __device__ __noinline__ void coop_modes(const BatchProblem &pr, int t, double *s
     case 4: coop_diag_t<6, RT, false>(pr.d, t, smem); break;
     case 5: coop_diag_t<6, RT, true>(pr.d, t, smem); break;
     case 6: coop_diag_t<8, RT, false>(pr.d, t, smem); break;
-    case 7: coop_diag_t<8, RT, true>(pr.d, t, smem); break;
-    case 8: coop_mixed_t<2, 32, false>(pr.m, t, smem); break;
-    case 9: coop_mixed_t<2, 32, true>(pr.m, t, smem); break;
-    case 10: coop_mixed_t<4, 32, false>(pr.m, t, smem); break;
-    case 11: coop_mixed_t<4, 32, true>(pr.m, t, smem); break;
-    case 12: coop_mixed_t<6, 32, false>(pr.m, t, smem); break;
-    case 13: coop_mixed_t<6, 32, true>(pr.m, t, smem); break;
-    case 14: coop_mixed_t<8, 32, false>(pr.m, t, smem); break;
-    default: coop_mixed_t<8, 32, true>(pr.m, t, smem); break;
+    default: coop_diag_t<8, RT, true>(pr.d, t, smem); break;
     }
 }
 
@@ -137,10 +123,6 @@ constexpr size_t coop_lds()
     m = cmax(m, sizeof(DiagShared<4, RT, true, false>));
     m = cmax(m, sizeof(DiagShared<6, RT, true, false>));
     m = cmax(m, sizeof(DiagShared<8, RT, true, false>));
-    m = cmax(m, sizeof(MixedShared<2, 32, true>));
-    m = cmax(m, sizeof(MixedShared<4, 32, true>));
-    m = cmax(m, sizeof(MixedShared<6, 32, true>));
-    m = cmax(m, sizeof(MixedShared<8, 32, true>));
     return m;
 }
 
@@ -203,7 +185,10 @@ __global__ __launch_bounds__(256, 2) void batch_coop_kernel(const BatchProblem *
 // Merged launches: one launch per stage over every task kind of the stage
 // (the per-XCD order of the fused variant, XCD-aware work-group mapping), the
 // task bodies inlined behind a switch, so small kinds share a launch with
-// large ones.  No waits: the launch boundaries order the stages.
+// large ones.  Mode solves of MIXED problems keep the staged variant's launches
+// (own_launch): their work-groups have sizes of their own, and a problem has
+// to come out the same, bit for bit, whichever variant the tuner picks.  No
+// waits: the launch boundaries order the stages.
 template <int KIND>
 __device__ __forceinline__ void merged_fft(const FftArgs &a, int L, int t, double *smem)
 {
@@ -249,15 +234,7 @@ __global__ __launch_bounds__(256) void batch_stage_modes(const BatchProblem *__r
     case 4: coop_diag_t<6, RT, false>(pr.d, e.y, smem); break;
     case 5: coop_diag_t<6, RT, true>(pr.d, e.y, smem); break;
     case 6: coop_diag_t<8, RT, false>(pr.d, e.y, smem); break;
-    case 7: coop_diag_t<8, RT, true>(pr.d, e.y, smem); break;
-    case 8: coop_mixed_t<2, 32, false>(pr.m, e.y, smem); break;
-    case 9: coop_mixed_t<2, 32, true>(pr.m, e.y, smem); break;
-    case 10: coop_mixed_t<4, 32, false>(pr.m, e.y, smem); break;
-    case 11: coop_mixed_t<4, 32, true>(pr.m, e.y, smem); break;
-    case 12: coop_mixed_t<6, 32, false>(pr.m, e.y, smem); break;
-    case 13: coop_mixed_t<6, 32, true>(pr.m, e.y, smem); break;
-    case 14: coop_mixed_t<8, 32, false>(pr.m, e.y, smem); break;
-    default: coop_mixed_t<8, 32, true>(pr.m, e.y, smem); break;
+    default: coop_diag_t<8, RT, true>(pr.d, e.y, smem); break;
     }
 }
 
@@ -341,6 +318,9 @@ using namespace hz;
 
 // ---- host side ---------------------------------------------------------------
 namespace {
+
+// Mode-solve kinds that are launched kind by kind in every variant.
+bool own_launch(int kind) { return kind >= 8; }
 
 // One element with Dirichlet faces in DIAG form, and a grid of the z-first
 // kernels (zfirst.hip): expand, filter, collect instead of the five stages.
@@ -510,23 +490,27 @@ int enqueue_t(hz_batch *b, const Variant &v, hipStream_t s)
     const int r = rt_index(RT);
     for (const auto &z : b->zlaunches)
         if (int st = launch_zf_list(b->d_zargs, b->d_zlist + z[2], z[3], z[0], z[1], s)) return st;
+    const auto &g = b->groups[r];
     if (v.fused == 2) {
         const auto &xo = b->h_coop_off[r];
         for (int st = 0; st < kStages; ++st) {
+            for (size_t i = 0; st == 2 && i + 1 < g.size(); ++i)
+                if (g[i][0] == 2 && own_launch(g[i][1]))
+                    launch_diag_list<RT>(s, b->d_probs, b->d_list[r] + g[i][2], g[i + 1][2] - g[i][2], g[i][1]);
             const int first = xo[(size_t)st * (kXcds + 1)], count = xo[(size_t)st * (kXcds + 1) + kXcds] - first;
             if (count == 0) continue;
             const int2 *list = b->d_coop_list[r] + first;
-            const dim3 g(count), blk(256);
+            const dim3 grid(count), blk(256);
             const int pass = st < 2 ? st : st - 1;
             const unsigned fl = (unsigned)merged_fft_lds();
             switch (st) {
-            case 0: hipLaunchKernelGGL((batch_stage_fft<FFT_R2C>), g, blk, fl, s, b->d_probs, list, pass); break;
-            case 1: hipLaunchKernelGGL((batch_stage_fft<FFT_C2C_FWD>), g, blk, fl, s, b->d_probs, list, pass); break;
+            case 0: hipLaunchKernelGGL((batch_stage_fft<FFT_R2C>), grid, blk, fl, s, b->d_probs, list, pass); break;
+            case 1: hipLaunchKernelGGL((batch_stage_fft<FFT_C2C_FWD>), grid, blk, fl, s, b->d_probs, list, pass); break;
             case 2:
-                hipLaunchKernelGGL((batch_stage_modes<RT>), g, blk, (unsigned)coop_lds<RT>(), s, b->d_probs, list);
+                hipLaunchKernelGGL((batch_stage_modes<RT>), grid, blk, (unsigned)coop_lds<RT>(), s, b->d_probs, list);
                 break;
-            case 3: hipLaunchKernelGGL((batch_stage_fft<FFT_C2C_INV>), g, blk, fl, s, b->d_probs, list, pass); break;
-            default: hipLaunchKernelGGL((batch_stage_fft<FFT_C2R>), g, blk, fl, s, b->d_probs, list, pass); break;
+            case 3: hipLaunchKernelGGL((batch_stage_fft<FFT_C2C_INV>), grid, blk, fl, s, b->d_probs, list, pass); break;
+            default: hipLaunchKernelGGL((batch_stage_fft<FFT_C2R>), grid, blk, fl, s, b->d_probs, list, pass); break;
             }
         }
         HZ_HIP(hipGetLastError());
@@ -542,7 +526,6 @@ int enqueue_t(hz_batch *b, const Variant &v, hipStream_t s)
         HZ_HIP(hipLaunchCooperativeKernel((const void *)batch_coop_kernel<RT>, dim3(b->coop_wgs[r] * b->cus),
                                           dim3(256), args, (unsigned)coop_lds<RT>(), s));
     } else {
-        const auto &g = b->groups[r];
         for (size_t i = 0; i + 1 < g.size(); ++i) {
             const int st = g[i][0], kind = g[i][1], first = g[i][2], count = g[i + 1][2] - first;
             if (count == 0) continue;  // e.g. only in-place length-1 passes (identities) of this kind
@@ -663,7 +646,7 @@ int build_lists(hz_batch *b, int rt)
         for (int x = 0; x < kXcds; ++x) {
             xo[(size_t)st * (kXcds + 1) + x] = (int)co.size();
             for (size_t gi = gr.size() - 1; gi-- > 0;) {
-                if (gr[gi][0] != st) continue;
+                if (gr[gi][0] != st || (st == 2 && own_launch(gr[gi][1]))) continue;
                 const long long first = gr[gi][2], count = gr[gi + 1][2] - first;
                 co.insert(co.end(), all.begin() + (first + count * x / kXcds),
                           all.begin() + (first + count * (x + 1) / kXcds));
@@ -671,7 +654,10 @@ int build_lists(hz_batch *b, int rt)
         }
         xo[(size_t)st * (kXcds + 1) + kXcds] = (int)co.size();
     }
-    if (co.size() != all.size()) return set_error(HZ_ERR_HIP, "batch: fused task order lost tasks");
+    size_t own = 0;
+    for (size_t gi = 0; gi + 1 < gr.size(); ++gi)
+        if (gr[gi][0] == 2 && own_launch(gr[gi][1])) own += gr[gi + 1][2] - gr[gi][2];
+    if (co.size() + own != all.size()) return set_error(HZ_ERR_HIP, "batch: fused task order lost tasks");
     (void)hipFree(b->d_coop_list[r]);
     (void)hipFree(b->d_coop_off[r]);
     b->d_coop_list[r] = nullptr;
@@ -757,7 +743,11 @@ int coop_residency(int *wgs)
 bool variant_usable(const hz_batch *b, int vi)
 {
     const Variant &v = kVariants[vi];
-    return !v.off && (v.fused != 1 || b->coop_wgs[rt_index(v.rt)] > 0);
+    if (v.off) return false;
+    if (v.fused != 1) return true;
+    for (int p = 0; p < b->n; ++p)  // the fused launch has no body for the kinds with launches of their own
+        if (own_launch(b->h_probs[p].dkind)) return false;
+    return b->coop_wgs[rt_index(v.rt)] > 0;
 }
 
 void free_batch(hz_batch *b)
