@@ -237,8 +237,9 @@ int hz_lu_solve_batched(const double *LU, const int *piv, double *b, int n, int 
  * staged (variants 4, 5: one launch per stage and kind of task, recorded in
  * a HIP graph that later solves replay, re-reading the buffer table when the
  * pointers change), merged (variants 8, 9: one launch per stage over every
- * task kind of the stage but the mode solves of MIXED plans, which are
- * launched as in 4 and 5; also recorded in a graph) and fused (variants 6, 7:
+ * task kind of the stage but the mode solves of MIXED plans and of short
+ * elements (N - 2 <= 32: several elements, Robin faces or periodic z), which
+ * are launched as in 4 and 5; also recorded in a graph) and fused (variants 6, 7:
  * ONE cooperative launch per solve, the five stages separated by grid
  * barriers; built but switched off and refused, since two of its GPU runs did
  * not finish).  The first solve of a batch shape times every usable variant

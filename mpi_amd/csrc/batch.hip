@@ -24,6 +24,7 @@
 // The autotuner times the usable variants (staged or fused, mode-solve tile
 // height 32 or 64 rows) on the first solve of a batch shape and keeps the
 // fastest.
+#include "diag_waves_body.h"
 #include "fft_body.h"
 #include "mixed_body.h"
 
@@ -44,7 +45,9 @@ struct BatchProblem {
     DiagArgs d;      // DIAG plans
     MixedArgs m;     // MIXED plans
     int ly, lx;      // transform lengths along y, x
-    int dkind;       // 2 * (NP / 32 - 1) + general (NP = 32, 64, 96, 128), + 8 for a MIXED plan
+    // 2 * (NP / 32 - 1) + general (NP = 32, 64, 96, 128), + 8 for a MIXED plan;
+    // 16, 17 (N - 2 to 16, to 32) for what diag_waves.hip solves
+    int dkind;
 };
 
 namespace {
@@ -80,14 +83,13 @@ __device__ __forceinline__ void coop_diag_t(const DiagArgs &a, int t, double *sm
     diag_tile<NJ, RT, GENERAL, false>(a, t, *reinterpret_cast<DiagShared<NJ, RT, GENERAL, false> *>(smem));
 }
 
-// A mode-solve task: tile t of the problem's DIAG kernel body (kinds 0-7; a
+// A mode-solve task: tile t of the problem's DIAG kernel body (kinds 0, 2-7; a
 // batch with other kinds is not run fused, see variant_usable).
 template <int RT>
 __device__ __noinline__ void coop_modes(const BatchProblem &pr, int t, double *smem)
 {
     switch (pr.dkind) {
     case 0: coop_diag_t<2, RT, false>(pr.d, t, smem); break;
-    case 1: coop_diag_t<2, RT, true>(pr.d, t, smem); break;
     case 2: coop_diag_t<4, RT, false>(pr.d, t, smem); break;
     case 3: coop_diag_t<4, RT, true>(pr.d, t, smem); break;
     case 4: coop_diag_t<6, RT, false>(pr.d, t, smem); break;
@@ -119,7 +121,7 @@ constexpr size_t coop_lds()
     size_t m = sizeof(double) * (256 + 2) * 16;  // transform tile, L = 256, W = 16
     m = cmax(m, sizeof(double) * (64 + 2) * 32);
     m = cmax(m, sizeof(double) * (16 + 2) * 64);
-    m = cmax(m, sizeof(DiagShared<2, RT, true, false>));
+    m = cmax(m, sizeof(DiagShared<2, RT, false, false>));
     m = cmax(m, sizeof(DiagShared<4, RT, true, false>));
     m = cmax(m, sizeof(DiagShared<6, RT, true, false>));
     m = cmax(m, sizeof(DiagShared<8, RT, true, false>));
@@ -185,8 +187,8 @@ __global__ __launch_bounds__(256, 2) void batch_coop_kernel(const BatchProblem *
 // Merged launches: one launch per stage over every task kind of the stage
 // (the per-XCD order of the fused variant, XCD-aware work-group mapping), the
 // task bodies inlined behind a switch, so small kinds share a launch with
-// large ones.  Mode solves of MIXED problems keep the staged variant's launches
-// (own_launch): their work-groups have sizes of their own, and a problem has
+// large ones.  Mode solves of MIXED problems and of diag_waves.hip's keep the
+// staged variant's launches (own_launch): their work-groups have sizes of their own, and a problem has
 // to come out the same, bit for bit, whichever variant the tuner picks.  No
 // waits: the launch boundaries order the stages.
 template <int KIND>
@@ -228,7 +230,6 @@ __global__ __launch_bounds__(256) void batch_stage_modes(const BatchProblem *__r
     const BatchProblem &pr = P[e.x];
     switch (pr.dkind) {
     case 0: coop_diag_t<2, RT, false>(pr.d, e.y, smem); break;
-    case 1: coop_diag_t<2, RT, true>(pr.d, e.y, smem); break;
     case 2: coop_diag_t<4, RT, false>(pr.d, e.y, smem); break;
     case 3: coop_diag_t<4, RT, true>(pr.d, e.y, smem); break;
     case 4: coop_diag_t<6, RT, false>(pr.d, e.y, smem); break;
@@ -299,6 +300,34 @@ __global__ __launch_bounds__(256) void batch_diag_list(const BatchProblem *__res
     __shared__ DiagShared<NJ, RT, GENERAL, false> sh;
     const int2 t = list[blockIdx.x];
     diag_tile<NJ, RT, GENERAL, false>(P[t.x].d, t.y, sh);
+}
+
+__device__ __forceinline__ DiagArgs global_args(DiagArgs a)
+{
+    a.spec = as_global(a.spec);
+    a.bc_re = as_global(a.bc_re);
+    a.bc_im = as_global(a.bc_im);
+    a.shift = as_global(a.shift);
+    a.mu = as_global(a.mu);
+    a.VinvT = as_global(a.VinvT);
+    a.VT = as_global(a.VT);
+    a.w0 = as_global(a.w0);
+    a.wN = as_global(a.wN);
+    a.r0 = as_global(a.r0);
+    a.rN = as_global(a.rN);
+    a.hom = as_global(a.hom);
+    a.closure = as_global(a.closure);
+    return a;
+}
+
+// Several elements, Robin faces or periodic z at N - 2 <= 32, as a single
+// solve takes them (diag_waves.hip).
+template <int NJ, int WR, int RB>
+__global__ __launch_bounds__(64 * NJ * WR, 4) void batch_diag_waves_list(const BatchProblem *__restrict__ P,
+                                                                         const int2 *__restrict__ list)
+{
+    const int2 t = list[blockIdx.x];
+    diag_waves_tile<NJ, WR, RB, false>(global_args(P[uniform(t.x)].d), uniform(t.y));
 }
 
 // One wave per 16 columns (mixed_waves_tile), 32 rows: 48 problems of 32 to 128
@@ -391,11 +420,10 @@ namespace {
 
 int rt_index(int rt) { return rt == 64 ? 1 : 0; }
 
-// Mode-solve tiles of a plan for DIAG tiles of `rt` rows (MIXED tiles have
-// 32).
-int mode_tiles(const hz_plan *pl, int rt)
+// Mode-solve tiles of a plan of that kind for DIAG tiles of `rt` rows.
+int mode_tiles(const hz_plan *pl, int kind, int rt)
 {
-    const int rows = pl->d.form == HZ_FORM_MIXED ? 32 : rt;
+    const int rows = kind >= 16 ? diag_waves_rows(pl->n) : kind >= 8 ? 32 : rt;
     const int fc_per_tile = rows / (2 * pl->ne);
     const int nfc = pl->nx * pl->M;
     return (nfc + fc_per_tile - 1) / fc_per_tile;
@@ -425,7 +453,10 @@ int fill_problems(hz_batch *b, const double *const *f, const double *const *gl, 
         q.ly = pl->ny;
         q.lx = pl->nx;
         const bool general = pl->ne > 1 || pl->d.alpha_l != 0.0 || pl->d.alpha_r != 0.0 || pl->d.periodic_z;
-        q.dkind = 2 * (diag_padded(pl->n) / 32 - 1) + (general ? 1 : 0) + (pl->d.form == HZ_FORM_MIXED ? 8 : 0);
+        const bool mixed = pl->d.form == HZ_FORM_MIXED;
+        q.dkind = general && !mixed && diag_waves_holds(pl->n, pl->ne)
+                      ? 16 + (pl->n > 16)
+                      : 2 * (diag_padded(pl->n) / 32 - 1) + (general ? 1 : 0) + (mixed ? 8 : 0);
     }
     return HZ_OK;
 }
@@ -468,13 +499,19 @@ template <int RT>
 void launch_diag_list(hipStream_t s, const BatchProblem *P, const int2 *list, int count, int kind)
 {
     const dim3 g(count), b(256);
+    if (kind >= 16) {
+        if (kind == 16)
+            hipLaunchKernelGGL((batch_diag_waves_list<1, 4, 2>), g, b, 0, s, P, list);
+        else
+            hipLaunchKernelGGL((batch_diag_waves_list<2, 2, 2>), g, b, 0, s, P, list);
+        return;
+    }
     if (kind >= 8) {
         launch_mixed_list(s, P, list, count, kind - 8);
         return;
     }
     switch (kind) {
     case 0: hipLaunchKernelGGL((batch_diag_list<2, RT, false>), g, b, 0, s, P, list); break;
-    case 1: hipLaunchKernelGGL((batch_diag_list<2, RT, true>), g, b, 0, s, P, list); break;
     case 2: hipLaunchKernelGGL((batch_diag_list<4, RT, false>), g, b, 0, s, P, list); break;
     case 3: hipLaunchKernelGGL((batch_diag_list<4, RT, true>), g, b, 0, s, P, list); break;
     case 4: hipLaunchKernelGGL((batch_diag_list<6, RT, false>), g, b, 0, s, P, list); break;
@@ -597,7 +634,7 @@ int build_lists(hz_batch *b, int rt)
         for (int st = 0; st < kStages; ++st) {
             if (b->zuse && z_first(b->plans[p])) continue;
             auto &v = by[{st, task_kind(b->h_probs[p], st)}];
-            int ntask = st == 2 ? mode_tiles(b->plans[p], rt) : 0;
+            int ntask = st == 2 ? mode_tiles(b->plans[p], b->h_probs[p].dkind, rt) : 0;
             if (st != 2) {  // transform passes: one entry per uniform-base tile
                 // The table is filled with null buffers here, so the face
                 // count is set from what hz_batch_solve always passes: both

@@ -129,6 +129,7 @@ int launch_diag_modes(const DiagArgs &a, hipStream_t s);
 // The same for several elements, Robin faces or periodic z at N - 2 <= 32
 // (diag_waves.hip); launch_diag_modes takes it where it holds.
 bool diag_waves_holds(int n, int ne);
+int diag_waves_rows(int n);  // of a tile
 int launch_diag_waves(const DiagArgs &a, hipStream_t s);
 
 

@@ -50,3 +50,11 @@ def test_mixed_batch(cuda):
     sizes = [(5, 1), (18, 8), (34, 3), (35, 1), (66, 2), (67, 5), (98, 1), (99, 4), (130, 1)]
     same_bits([(nx, ny, N, ne, faces) for (nx, ny) in ((32, 16), (1, 32)) for N, ne in sizes
                for faces in ("dirichlet", "robin", "periodic")], "mixed")
+
+
+def test_diag_batch_general(cuda):
+    """DIAG problems of several elements, Robin faces or periodic z, N - 2 at
+    the edges of the column tiles (short elements have a kernel of their own)."""
+    sizes = [(3, 1), (5, 16), (9, 8), (18, 16), (19, 3), (34, 8), (35, 1), (66, 2), (67, 1), (99, 4), (130, 1)]
+    same_bits([(nx, ny, N, ne, faces) for (nx, ny) in ((32, 16), (1, 32)) for N, ne in sizes
+               for faces in ("robin", "periodic", "dirichlet")[:3 if ne > 1 else 2]], "diag")
