@@ -244,8 +244,17 @@ int hz_lu_solve_batched(const double *LU, const int *piv, double *b, int n, int 
  * barriers; built but switched off and refused, since two of its GPU runs did
  * not finish).  The first solve of a batch shape times every usable variant
  * and keeps the fastest.  Variants 0-3 are refused (an earlier fused design,
- * removed).  One-element Dirichlet DIAG problems with nx, ny in [32, 256] run
- * ahead of the rest in three launches of their own, in every variant.
+ * removed).
+ * One-element Dirichlet DIAG problems with nx, ny in [32, 256] take three
+ * stages of their own, ahead of the rest and alike in every variant, if they
+ * have together at least one tile of 64 (x, y) points per compute unit (sum of
+ * nx ny / 64): one launch, then one for all grids of at most 16,384 points with
+ * ny < 256 and one for each larger grid, then one launch.  So whether a
+ * problem goes this way depends on the whole batch; its result then agrees
+ * with its plan's own solve to rounding (1e-13 of the largest value), and has
+ * the same bits where that solve goes this way too.  Every other problem has
+ * the bits of its plan's own solve.  A given batch gives the same bits in
+ * every variant and in every solve.
  * Enqueued on `stream`; a plan in a batch must not be used by another solve
  * while the batch runs. */
 typedef struct hz_batch hz_batch;

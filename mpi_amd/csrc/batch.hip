@@ -585,7 +585,10 @@ int enqueue_t(hz_batch *b, const Variant &v, hipStream_t s)
 // points a side and 17 to 129 along z (317 MB) take 400 us, 600 in five stages.
 // Used from one tile per CU on (16 of 32 x 32 x 17: 78 us either way; x 129 80
 // against 96): on fewer, the five stages' many short work-groups fill the chip
-// better.
+// better.  A problem's route, and with it its low bits, so depend on the rest of
+// its batch; taking the single solve's route instead runs the two halves of a
+// batch one after the other (8 / 64 problems of 32 to 128 points a side 92 ->
+// 133, 493 -> 633 us).
 int build_zlists(hz_batch *b)
 {
     int tiles = 0;

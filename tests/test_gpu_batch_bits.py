@@ -58,3 +58,39 @@ def test_diag_batch_general(cuda):
     sizes = [(3, 1), (5, 16), (9, 8), (18, 16), (19, 3), (34, 8), (35, 1), (66, 2), (67, 1), (99, 4), (130, 1)]
     same_bits([(nx, ny, N, ne, faces) for (nx, ny) in ((32, 16), (1, 32)) for N, ne in sizes
                for faces in ("robin", "periodic", "dirichlet")[:3 if ne > 1 else 2]], "diag")
+
+
+def test_diag_batch_dirichlet_five_stages(cuda):
+    """One-element Dirichlet DIAG problems that stay on the five stages in every
+    variant: sides of 16, and so few tiles of larger grids that the z-first
+    kernels (whose bits differ) are not taken; every padded size."""
+    Ns = (3, 17, 33, 34, 35, 65, 66, 67, 97, 98, 99, 129, 130)
+    sides = ((16, 256), (256, 16), (16, 16), (64, 16), (16, 128), (1, 64), (1, 1))
+    same_bits([(nx, ny, N, 1, "dirichlet") for nx, ny in sides for N in Ns], "diag")
+    same_bits([(32, 32, N, 1, "dirichlet") for N in Ns] + [(32, 64, 130, 1, "dirichlet")], "diag", [[0], [12, 13]])
+
+
+def test_diag_batch_z_first_bits(cuda):
+    """A batch whose one-element Dirichlet problems go z-first: the same bits in
+    every variant and in the next solve; those of the single solve where that
+    goes z-first too, else equal to rounding (1e-13)."""
+    import torch
+    from mpi_amd.solver import BatchSolver
+    specs = [(nx, ny, N, 1, "dirichlet") for nx, ny in ((32, 32), (32, 256), (64, 64), (128, 64), (128, 128), (256, 32))
+             for N in (5, 34, 67, 130)] + [(16, 32, 33, 1, "dirichlet"), (32, 16, 9, 2, "robin")]
+    plans, fs, gs, want = problems(specs, "diag")
+    b = BatchSolver(plans)
+    first = None
+    for variant in VARIANTS * 2:
+        b.force_variant(variant)
+        us = b.solve(fs, gs, gs)
+        b.status()
+        first = first or [u.clone() for u in us]
+        assert all(torch.equal(u, v) for u, v in zip(us, first)), variant
+    b.close()
+    for spec, p, u, w, f, g in zip(specs, plans, first, want, fs, gs):
+        p.profile(True)
+        p.solve(f, g, g)
+        alone = "xy_filter" in p.profile_read()[0]
+        assert torch.equal(u, w) if alone or 16 in spec[:2] else float((u - w).abs().max() / w.abs().max()) <= 1e-13
+        p.close()
