@@ -1087,7 +1087,8 @@ __global__ __launch_bounds__(64) void lu_solve_wave_kernel(const double *__restr
         if (lane + 64 * a < n) xb[lane + 64 * a] = x[a];
 }
 
-// The same for systems of more than 128 (one thread per system).
+// The same, one thread per system: orders above 128, and the small systems of
+// lu_solve_by_thread.
 __global__ void lu_solve_kernel(const double *LU, const int *piv, double *b, int n, int count)
 {
 #pragma clang fp contract(off)
@@ -1159,16 +1160,38 @@ int launch_lu_factor(const LuFactorArgs &a, hipStream_t s)
     return set_error(HZ_ERR_UNSUPPORTED, "batched FP64 LU supports n <= 128");
 }
 
+// One thread per system where a wave has too little to do.  Its rows are read
+// uncoalesced, but up to order 6 a system is a few cache lines; to order 10 it
+// is the faster while there are threads to fill the chip and the matrices stay
+// in the caches.  Measured, us, one thread | one wave per system: order 2, 65,536
+// systems 7 | 31, 1,048,576 14 | 438; order 6, 1,024 7 | 7, 65,536 32 | 96,
+// 524,288 356 | 363; order 8, 8,192 14 | 11, 24,576 15 | 26, 131,072 102 | 118,
+// 262,144 375 | 243; order 10, 8,192 18 | 13, 24,576 20 | 27, 131,072 254 | 142;
+// order 12, 24,576 28 | 27.
+static bool lu_solve_by_thread(int n, int count)
+{
+    return n <= 6 || (n <= 10 && count >= 1600 * (n - 2) && (long long)count * n * n <= 1 << 23);
+}
+
 int launch_lu_solve(const double *LU, const int *piv, double *b, int n, int count, hipStream_t s)
 {
     if (count <= 0) return HZ_OK;
-    if (n <= 64)
-        hipLaunchKernelGGL(lu_solve_wave_kernel<1>, dim3(count), dim3(64), 0, s, LU, piv, b, n);
-    else if (n <= 128)
-        hipLaunchKernelGGL(lu_solve_wave_kernel<2>, dim3(count), dim3(64), 0, s, LU, piv, b, n);
-    else
+    if (n > 128 || lu_solve_by_thread(n, count)) {
         hipLaunchKernelGGL(lu_solve_kernel, dim3((count + 63) / 64), dim3(64), 0, s, LU, piv, b, n, count);
-    HZ_HIP(hipGetLastError());
+        HZ_HIP(hipGetLastError());
+        return HZ_OK;
+    }
+    // a launch has fewer than 2^32 threads
+    for (long long first = 0; first < count; first += 1 << 25) {
+        const dim3 grid((unsigned)std::min<long long>(count - first, 1 << 25));
+        const double *A = LU + first * n * n;
+        const int *p = piv + first * (n - 1);
+        if (n <= 64)
+            hipLaunchKernelGGL(lu_solve_wave_kernel<1>, grid, dim3(64), 0, s, A, p, b + first * n, n);
+        else
+            hipLaunchKernelGGL(lu_solve_wave_kernel<2>, grid, dim3(64), 0, s, A, p, b + first * n, n);
+        HZ_HIP(hipGetLastError());
+    }
     return HZ_OK;
 }
 
