@@ -1163,11 +1163,11 @@ int launch_lu_factor(const LuFactorArgs &a, hipStream_t s)
 // One thread per system where a wave has too little to do.  Its rows are read
 // uncoalesced, but up to order 6 a system is a few cache lines; to order 10 it
 // is the faster while there are threads to fill the chip and the matrices stay
-// in the caches.  Measured, us, one thread | one wave per system: order 2, 65,536
-// systems 7 | 31, 1,048,576 14 | 438; order 6, 1,024 7 | 7, 65,536 32 | 96,
-// 524,288 356 | 363; order 8, 8,192 14 | 11, 24,576 15 | 26, 131,072 102 | 118,
-// 262,144 375 | 243; order 10, 8,192 18 | 13, 24,576 20 | 27, 131,072 254 | 142;
-// order 12, 24,576 28 | 27.
+// in the caches.  Measured, us, one thread | one wave per system: order 2,
+// 131,072 systems 7 | 58, 1,048,576 14 | 438; order 6, 1,024 7 | 7, 65,536
+// 17 | 51, 524,288 364 | 370; order 8, 8,192 14 | 11, 24,576 15 | 26, 131,072
+// 103 | 118, 262,144 359 | 233; order 10, 8,192 18 | 13, 24,576 24 | 31, 131,072
+// 254 | 142; order 12, 24,576 38 | 36.
 static bool lu_solve_by_thread(int n, int count)
 {
     return n <= 6 || (n <= 10 && count >= 1600 * (n - 2) && (long long)count * n * n <= 1 << 23);
