@@ -29,6 +29,30 @@ constexpr int kDerivCols = 64;
 
 int deriv_rows(int N) { return (N + 16) / 17 < (N + 15) / 16 ? 17 : 16; }
 
+// Few outputs: one thread per output, so that they spread over the chip (a tile
+// of 64 columns is one work-group, whose waves run N steps of 17 products each).
+// Eight loads of each operand in flight: one at a time, 256 columns of 129 took
+// 17 us against 7.5.
+__global__ __launch_bounds__(256) void derivative_few_kernel(const double *__restrict__ DT, int N, int KP, int total,
+                                                             const double *__restrict__ u, double *__restrict__ out)
+{
+#pragma clang fp contract(off)
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= total) return;
+    const int k = idx % N;
+    const double *uc = u + (idx - k);
+    double acc = 0.0;
+#pragma unroll 8
+    for (int p = 0; p < N; ++p) acc += DT[p * KP + k] * uc[p];
+    out[idx] = acc;
+}
+
+// Where that is the faster: to four work-groups of outputs per CU.  Measured, us,
+// one thread per output | tiles: 1 column of N = 66 7 | 11, of 257 12 | 76; 256
+// columns of 129 7.5 | 26.5; 2,048 of 128 23.5 | 37.4, of 129 29.8 | 26.9; 4,096 of
+// 64 13 | 20, of 66 16.5 | 14.4; 8,192 of 32 7.7 | 11.7, of 33 9.7 | 8.3.
+bool derivative_few(int N, long long ncols) { return ncols * N <= 1 << 18; }
+
 template <int R>
 __global__ __launch_bounds__(1024) void derivative_kernel(const double *__restrict__ DT, int N, int KP, long long ncols,
                                                          const double *__restrict__ u, double *__restrict__ out)
@@ -255,7 +279,12 @@ int launch_derivative(const double *DT, int N, long long ncols, const double *u,
     if (waves > 16 || lds > 160 * 1024 || blocks > 0x7fffffffLL)
         return set_error(HZ_ERR_UNSUPPORTED, "derivative: field too large");
     const dim3 grid((unsigned)blocks), block(64 * waves);
-    if (R == 17)
+    const long long total = ncols * N;
+    // (outputs that overlap the inputs: a tile has read all of its columns before it stores)
+    if (derivative_few(N, ncols) && (out + total <= u || u + total <= out)) {
+        hipLaunchKernelGGL(derivative_few_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, DT, N,
+                           strips * R, (int)total, u, out);
+    } else if (R == 17)
         hipLaunchKernelGGL((derivative_kernel<17>), grid, block, (unsigned)lds, s, DT, N, strips * R, ncols, u, out);
     else
         hipLaunchKernelGGL((derivative_kernel<16>), grid, block, (unsigned)lds, s, DT, N, strips * R, ncols, u, out);

@@ -72,3 +72,42 @@ def test_lu_solve_of_more_systems_than_one_launch_holds(cuda):
     lu_solve_batched(LU, pv, x)
     assert torch.equal(x[:count // 1000 * 1000].view(-1, 1000, n),
                        want.expand(count // 1000, 1000, n)) and torch.equal(x[-(count % 1000):], want[:count % 1000])
+
+
+@pytest.mark.parametrize("N", [129, 257])
+def test_derivative_z_of_few_columns_is_short(cuda, N):
+    """One column (a 1-D problem's field) is spread over the chip: at most 0.6 of
+    the time of 16,384 columns, one tile per CU."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    took = []
+    for side in (1, 128):
+        plan = HelmholtzPlan(side, side, N, 1, form="diag")
+        u = torch.randn((1, side, side, N), dtype=torch.float64, device="cuda")
+        out = torch.empty_like(u)
+        took.append(best_us(lambda: plan.derivative_z(u, 1, out=out)))
+        plan.close()
+    assert took[0] <= 0.6 * took[1], took
+
+
+@pytest.mark.parametrize("nx,ny,N", [(1, 1, 3), (1, 1, 258), (16, 64, 256), (32, 32, 257), (64, 64, 64), (64, 64, 65),
+                                     (128, 128, 16), (128, 128, 17)])
+def test_derivative_z_few_and_many_outputs(cuda, nx, ny, N):
+    """One thread per output (to 2^18 outputs), tiles of 64 columns above and
+    where the output is the input: the reference's products and sums in its
+    order, bit for bit."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    plan = HelmholtzPlan(nx, ny, N, 1, form="diag")
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    u = torch.randn((1, nx, ny, N), dtype=torch.float64, device="cuda", generator=gen)
+    for order, D in zip((1, 2), plan.operators()):
+        Dd = torch.from_numpy(np.ascontiguousarray(D)).cuda()
+        want = torch.zeros_like(u)
+        for p in range(N):  # p ascending, every product rounded before it is added
+            want = want + Dd[:, p] * u[..., p:p + 1]
+        assert torch.equal(plan.derivative_z(u, order, out=torch.empty_like(u)), want)
+        same = u.clone()
+        plan.derivative_z(same, order, out=same)
+        assert torch.equal(same, want)
+    plan.close()
