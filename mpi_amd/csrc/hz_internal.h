@@ -70,7 +70,7 @@ int launch_fft(int L, FftKind kind, const FftArgs &a, hipStream_t s);
 // Lane widths offered for length L (autotuned per plan); returns the count.
 int fft_width_choices(int L, int *w, int max);
 
-// Arguments of the plain-LU mode kernel (lu_modes.hip).
+// Arguments of the plain-LU mode kernels (lu_modes.hip, lu.hip).
 struct LuModeArgs {
     int nx, ny, M, K, N, n, ne;
     long long xs;            // spectrum x-row stride (>= M * K)
@@ -90,7 +90,8 @@ struct LuModeArgs {
     int cols;                // instance column capacity (lu_modes_shapes); 0 = the smallest
 };
 int launch_lu_modes(const LuModeArgs &a, int modes, hipStream_t s);
-int launch_lu_modes_above_64(const LuModeArgs &a, int modes, hipStream_t s);  // N - 2 > 64
+// lu.hip's kernel, by column capacity; at most 30 right-hand sides of elements.
+int launch_lu_modes_stepwise(const LuModeArgs &a, int cols, int modes, hipStream_t s);
 // The mode kernels' LDS limit on the current device (once per plan).
 int lu_modes_prepare();
 // Column capacities (16, 32, 64, 128) of the mode-kernel instances that hold

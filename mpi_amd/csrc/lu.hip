@@ -1,6 +1,7 @@
-// lu.hip -- the reference algorithm per (|kx|,|ky|) mode for N - 2 above 64
-// (smaller operators: lu_modes.hip): one work-group per mode, the whole
-// augmented system resident in registers; and the standalone batched LU.
+// lu.hip -- the reference algorithm per (|kx|,|ky|) mode for N - 2 above 64, and
+// for small operators of few modes (the rest: lu_modes.hip, which chooses): one
+// work-group per mode, the whole augmented system resident in registers; and the
+// standalone batched LU.
 //
 // For mode (iw, jw) the work-group
 //   1. assembles A = Dzz_int - sigma I (or the caller's operator) and the
@@ -1117,10 +1118,15 @@ __global__ void lu_solve_kernel(const double *LU, const int *piv, double *b, int
     }
 }
 
-template <int NR>
+template <int RB, int CB>
 int launch_modes_t(const LuModeArgs &a, int modes, hipStream_t s)
 {
-    hipLaunchKernelGGL((lu_modes_kernel<2, 32, NR, 4>), dim3(modes), dim3(WAVE * 4), 0, s, a);
+    const int nr = (2 + rhs_per_element(a.nx) * a.ne + 3) / 4;  // right-hand sides per wave
+    if (nr > 8) return set_error(HZ_ERR_UNSUPPORTED, "PLAIN_LU form: too many elements for the stepwise kernel");
+    if (nr <= 2)
+        hipLaunchKernelGGL((lu_modes_kernel<RB, CB, 2, 4>), dim3(modes), dim3(WAVE * 4), 0, s, a);
+    else
+        hipLaunchKernelGGL((lu_modes_kernel<RB, CB, 8, 4>), dim3(modes), dim3(WAVE * 4), 0, s, a);
     HZ_HIP(hipGetLastError());
     return HZ_OK;
 }
@@ -1135,10 +1141,14 @@ int launch_factor_t(const LuFactorArgs &a, hipStream_t s)
 
 }  // namespace
 
-int launch_lu_modes_above_64(const LuModeArgs &a, int modes, hipStream_t s)
+int launch_lu_modes_stepwise(const LuModeArgs &a, int cols, int modes, hipStream_t s)
 {
-    const int nr = (2 + rhs_per_element(a.nx) * a.ne + 3) / 4;  // right-hand sides per wave
-    return nr <= 2 ? launch_modes_t<2>(a, modes, s) : launch_modes_t<8>(a, modes, s);
+    switch (cols) {
+    case 16: return launch_modes_t<1, 4>(a, modes, s);
+    case 32: return launch_modes_t<1, 8>(a, modes, s);
+    case 64: return launch_modes_t<1, 16>(a, modes, s);
+    default: return launch_modes_t<2, 32>(a, modes, s);
+    }
 }
 
 int launch_lu_factor(const LuFactorArgs &a, hipStream_t s)

@@ -48,8 +48,9 @@
 // 78 -> 35, 128^2 with 8 of 17 243 -> 64, 64^2 with 4 of 33 88 -> 42.
 // Above 64 rows a work-group needs 8 waves of 179 registers, one per CU, and
 // the other kernel is the faster (127 rows: 5.7 ms against 8.2 and more):
-// launch_lu_modes sends N - 2 > 64 there.  The instance of 8 tiles serves a
-// caller who pins the largest shape for a small operator.
+// launch_lu_modes sends N - 2 > 64 there, and small operators of few modes
+// (stepwise).  The instance of 8 tiles serves a caller who pins the largest
+// shape for a small operator.
 #include "hz_internal.h"
 #include "sweep.h"
 #include "wave_ops.h"
@@ -815,6 +816,32 @@ int lu_modes_shapes(int nx, int n, int ne, int *cols, int max)
     return k;
 }
 
+// Small operators on few modes: lu.hip's kernel, whose four waves of a mode start
+// and end it sooner and pay by the step, where a panel here costs the same for
+// any number of columns: N - 2 just above a multiple of 16, or little of either.
+// `c` right-hand sides of elements.  The rule follows from the plan's sizes
+// alone, so that every instance gives the same bits.  Measured, us a solve,
+// stepwise | panels, one element: 256^2 x 3 79 | 99, x 4 93 | 104, x 5 116 | 115;
+// 64^2 x 3 20 | 26, x 9 28.6 | 29.4, x 10 29.8 | 29.6, x 19 46 | 43; 1 x 64 x 9
+// 15 | 19, x 16 21.3 | 21.8, x 18 22.7 | 21.6, x 19 25 | 29, x 26 30.9 | 32.1,
+// x 34 36.9 | 33.9, x 35 39.9 | 41.1.
+static bool stepwise(int n, int c, int modes)
+{
+    // up to n rows: at most c such right-hand sides, and `work` of them over all
+    // modes (`work4` where a mode has four or fewer)
+    static const struct {
+        int n, c;
+        long long work, work4;
+    } lines[] = {{1, 30, 68000, 1LL << 62}, {2, 30, 24000, 1LL << 62}, {3, 30, 14000, 48000}, {4, 28, 9200, 22000},
+                 {5, 28, 6800, 6800},       {6, 24, 4800, 4800},       {7, 20, 4400, 4400},   {8, 16, 2400, 2400},
+                 {10, 10, 1200, 1200},      {12, 6, 400, 400},         {14, 4, 140, 140},     {16, 0, 0, 0},
+                 {18, 10, 1200, 1200},      {20, 6, 480, 480},         {22, 6, 400, 400},     {26, 4, 140, 140},
+                 {32, 0, 0, 0},             {35, 4, 140, 140}};
+    for (const auto &l : lines)
+        if (n <= l.n) return c <= l.c && (long long)modes * c <= (c <= 4 ? l.work4 : l.work);
+    return false;
+}
+
 int launch_lu_modes(const LuModeArgs &a, int modes, hipStream_t s)
 {
     if (int st = lu_modes_check(a.nx, a.n, a.ne)) return st;
@@ -824,7 +851,8 @@ int launch_lu_modes(const LuModeArgs &a, int modes, hipStream_t s)
     bool held = false;
     for (int i = 0; i < k && i < 4; ++i) held = held || c[i] == cols;
     if (!held) return set_error(HZ_ERR_ARG, "PLAIN_LU form: the mode-kernel shape does not hold this plan");
-    if (a.n > 64) return launch_lu_modes_above_64(a, modes, s);
+    if (a.n > 64 || stepwise(a.n, rhs_per_element(a.nx) * a.ne, modes))
+        return launch_lu_modes_stepwise(a, cols, modes, s);
     switch (cols) {
     case 16: return launch_modes_t<1>(a, modes, s);
     case 32: return launch_modes_t<2>(a, modes, s);

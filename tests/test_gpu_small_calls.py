@@ -111,3 +111,95 @@ def test_derivative_z_few_and_many_outputs(cuda, nx, ny, N):
         plan.derivative_z(same, order, out=same)
         assert torch.equal(same, want)
     plan.close()
+
+
+@pytest.mark.parametrize("N", [3, 4])
+def test_plain_smallest_operators_are_short(cuda, N):
+    """The reference algorithm with one or two interior nodes against seven: at
+    most three quarters of the time (16-column panels cost nearly the same)."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    took = []
+    for n in (N, 9):
+        plan = HelmholtzPlan(128, 128, n, 1, lam=3.0, form="plain")
+        f = torch.randn((128, 128, n), dtype=torch.float64, device="cuda")
+        g = torch.randn((128, 128), dtype=torch.float64, device="cuda")
+        u = plan.empty_field()
+        took.append(best_us(lambda: plan.solve(f, g, g, out=u)))
+        plan.close()
+    assert took[0] <= 0.75 * took[1], took
+
+
+@pytest.mark.parametrize("nx,ny,N,ne", [(1, 1, 3, 1), (256, 64, 3, 4), (128, 128, 4, 1), (128, 128, 4, 2),
+                                        (128, 256, 5, 1), (256, 256, 5, 1), (128, 128, 6, 1), (256, 128, 6, 1),
+                                        (64, 64, 7, 1), (128, 64, 7, 1), (1, 64, 8, 12), (1, 64, 8, 13),
+                                        (64, 32, 10, 1), (64, 64, 10, 1), (32, 32, 12, 1), (64, 32, 12, 1),
+                                        (16, 16, 14, 1), (32, 32, 14, 1), (1, 64, 16, 1), (1, 128, 16, 2),
+                                        (32, 32, 20, 1), (64, 32, 20, 1), (16, 16, 24, 1), (1, 64, 35, 1),
+                                        (1, 64, 37, 1), (16, 16, 37, 1)])
+def test_plain_both_kernels_at_the_line_between_them(cuda, nx, ny, N, ne):
+    """Sizes on either side of the rule that sends small operators of few modes
+    to the stepwise kernel: against the oracle within twice its rounding spread
+    (or 1e-12), every instance with the same bits."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    from oracle import pyoracle as po
+    lam = 3.0
+    geo = dict(xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2)
+    plan = HelmholtzPlan(nx, ny, N, ne, lam=lam, form="plain", **geo)
+    r = np.random.default_rng(N + ne)
+    f = r.standard_normal((nx, ny, plan.nz))
+    g = [r.standard_normal((nx, ny)) for _ in range(2)]
+    dev = [torch.from_numpy(v).cuda() for v in (f, *g)]
+    desc = po.make_desc(nx, ny, ne * N, N, size=1, lam=lam, **geo)
+    uo, uf = po.solve(desc, f, *g), po.solve(desc, f, *g, fma=True)
+    bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+    u = plan.solve(*dev)
+    plan.status()
+    assert np.abs(u.cpu().numpy() - uo).max() <= bar * np.abs(uo).max()
+    for cols in plan.diag_candidates():
+        plan.set_diag_tile(cols)
+        assert torch.equal(plan.solve(*dev), u)
+        plan.status()
+    plan.close()
+
+
+@pytest.mark.parametrize("N", [7, 9, 11, 16, 19, 24, 35])
+@pytest.mark.parametrize("scale", ["unit", "rows", "small", "huge"])
+def test_plain_panels_of_small_operators_on_many_modes(cuda, N, scale):
+    """The panel kernel's first columns and a second panel of few, on operators
+    of their own for every mode that exchange rows at almost every step (rows of
+    very different scale; scales whose reciprocals leave the ordinary range): u
+    per mode from numpy's solve.  Elimination with partial pivoting: n eps times
+    the condition, and a growth of 8; a mode with a zero column is singular."""
+    import torch
+    from mpi_amd._lib import HzError
+    from mpi_amd.solver import HelmholtzPlan
+    nx, ny, n = 128, 64, N - 2
+    plan = HelmholtzPlan(nx, ny, N, 1, form="plain")
+    M = ny // 2 + 1
+    r = np.random.default_rng(N)
+    A = r.standard_normal((nx // 2 + 1, M, n, n)) + 2.0 * np.eye(n)
+    s = {"unit": np.ones(n), "rows": 10.0 ** r.integers(-6, 7, n), "small": np.full(n, 2.0 ** -600),
+         "huge": np.full(n, 2.0 ** 1000)}[scale]
+    w = {"unit": 1.0, "rows": 1.0, "small": 2.0 ** -600, "huge": 2.0 ** 900}[scale]  # of the right-hand side
+    f = r.standard_normal((nx, ny, N)) * w
+    dev = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()  # noqa: E731
+    zero = dev(np.zeros((nx, ny)))
+    op = (s[:, None] * A).reshape(-1, n, n)
+    u = plan.solve_operators(dev(f), zero, zero, op_full=dev(op)).cpu().numpy()
+    plan.status()
+    F = np.fft.rfft2(f[:, :, 1:-1] / w, axes=(0, 1))
+    ix = np.minimum(np.arange(nx), nx - np.arange(nx))
+    As = A[ix]                                              # [nx, M, n, n]
+    ratio = s / w
+    W = np.linalg.solve(As, (F / ratio)[..., None])[..., 0]
+    want = np.fft.irfft2(W, s=(nx, ny), axes=(0, 1))
+    # a mode's error, n eps cond |u|, and its sum over the modes in the transform back
+    tol = 8 * n * 2.0 ** -52 * (np.linalg.cond(As) * np.abs(W).max(-1)).sum() * 2 / (nx * ny)
+    assert np.abs(u[:, :, 1:-1] - want).max() <= tol
+    op[7, :, n // 2] = 0.0
+    plan.solve_operators(dev(f), zero, zero, op_full=dev(op))
+    with pytest.raises(HzError):
+        plan.status()
+    plan.close()
