@@ -21,10 +21,10 @@ struct Lines {
     static constexpr int R1 = L >= 128 ? 16 : 8, R2 = L / R1, W = 256 / R2;
 };
 
+// (out may be u: a work-group stores its lines after it has read them whole)
 template <int L, int ORDER>
-__global__ __launch_bounds__(256, 4) void derivative_lines(const double *__restrict__ u, double *__restrict__ out,
-                                                           long long nbatch, long long lanes, long long bs,
-                                                           long long ps, double len,
+__global__ __launch_bounds__(256, 4) void derivative_lines(const double *u, double *out, long long nbatch,
+                                                           long long lanes, long long bs, long long ps, double len,
                                                            const double2 *__restrict__ tw)
 {
     constexpr int R1 = Lines<L>::R1, R2 = Lines<L>::R2, W = Lines<L>::W, NL = R1 / R2;

@@ -24,7 +24,8 @@ namespace {
 //
 // R = 17 where it saves a strip (N = 2^m + 1, the usual GLL sizes, would leave
 // one row to a strip of 16 that costs as much as the others, and an odd number
-// of waves to the four SIMDs).
+// of waves to the four SIMDs).  The output may be the input: a work-group stores
+// its columns after it has read them.
 constexpr int kDerivCols = 64;
 
 int deriv_rows(int N) { return (N + 16) / 17 < (N + 15) / 16 ? 17 : 16; }
@@ -55,7 +56,7 @@ bool derivative_few(int N, long long ncols) { return ncols * N <= 1 << 18; }
 
 template <int R>
 __global__ __launch_bounds__(1024) void derivative_kernel(const double *__restrict__ DT, int N, int KP, long long ncols,
-                                                         const double *__restrict__ u, double *__restrict__ out)
+                                                         const double *u, double *out)
 {
 #pragma clang fp contract(off)
     extern __shared__ double dtile[];
