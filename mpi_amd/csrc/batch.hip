@@ -46,7 +46,8 @@ struct BatchProblem {
     MixedArgs m;     // MIXED plans
     int ly, lx;      // transform lengths along y, x
     // 2 * (NP / 32 - 1) + general (NP = 32, 64, 96, 128), + 8 for a MIXED plan;
-    // 16, 17 (N - 2 to 16, to 32) for what diag_waves.hip solves
+    // 16, 17 (N - 2 to 16, to 32) for what diag_waves.hip solves, 18 for a MIXED
+    // plan of mixed_by_four_waves
     int dkind;
 };
 
@@ -330,6 +331,14 @@ __global__ __launch_bounds__(64 * NJ * WR, 4) void batch_diag_waves_list(const B
     diag_waves_tile<NJ, WR, RB, false>(global_args(P[uniform(t.x)].d), uniform(t.y));
 }
 
+__global__ __launch_bounds__(256, 2) void batch_mixed_tile_list(const BatchProblem *__restrict__ P,
+                                                                const int2 *__restrict__ list)
+{
+    __shared__ MixedShared<6, 32, true> sh;
+    const int2 t = list[blockIdx.x];
+    mixed_tile<6, 32, true>(P[t.x].m, t.y, sh);
+}
+
 // One wave per 16 columns (mixed_waves_tile), 32 rows: 48 problems of 32 to 128
 // points a side 618 us, with mixed_tile's four waves a tile 877.
 template <int NJ, bool GENERAL>
@@ -423,7 +432,7 @@ int rt_index(int rt) { return rt == 64 ? 1 : 0; }
 // Mode-solve tiles of a plan of that kind for DIAG tiles of `rt` rows.
 int mode_tiles(const hz_plan *pl, int kind, int rt)
 {
-    const int rows = kind >= 16 ? diag_waves_rows(pl->n) : kind >= 8 ? 32 : rt;
+    const int rows = kind == 16 || kind == 17 ? diag_waves_rows(pl->n) : kind >= 8 ? 32 : rt;
     const int fc_per_tile = rows / (2 * pl->ne);
     const int nfc = pl->nx * pl->M;
     return (nfc + fc_per_tile - 1) / fc_per_tile;
@@ -454,9 +463,12 @@ int fill_problems(hz_batch *b, const double *const *f, const double *const *gl, 
         q.lx = pl->nx;
         const bool general = pl->ne > 1 || pl->d.alpha_l != 0.0 || pl->d.alpha_r != 0.0 || pl->d.periodic_z;
         const bool mixed = pl->d.form == HZ_FORM_MIXED;
-        q.dkind = general && !mixed && diag_waves_holds(pl->n, pl->ne)
-                      ? 16 + (pl->n > 16)
-                      : 2 * (diag_padded(pl->n) / 32 - 1) + (general ? 1 : 0) + (mixed ? 8 : 0);
+        if (mixed && mixed_by_four_waves(pl->n, pl->ne, pl->nx * pl->M))
+            q.dkind = 18;
+        else if (general && !mixed && diag_waves_holds(pl->n, pl->ne))
+            q.dkind = 16 + (pl->n > 16);
+        else
+            q.dkind = 2 * (diag_padded(pl->n) / 32 - 1) + (general ? 1 : 0) + (mixed ? 8 : 0);
     }
     return HZ_OK;
 }
@@ -500,7 +512,9 @@ void launch_diag_list(hipStream_t s, const BatchProblem *P, const int2 *list, in
 {
     const dim3 g(count), b(256);
     if (kind >= 16) {
-        if (kind == 16)
+        if (kind == 18)
+            hipLaunchKernelGGL(batch_mixed_tile_list, g, b, 0, s, P, list);
+        else if (kind == 16)
             hipLaunchKernelGGL((batch_diag_waves_list<1, 4, 2>), g, b, 0, s, P, list);
         else
             hipLaunchKernelGGL((batch_diag_waves_list<2, 2, 2>), g, b, 0, s, P, list);

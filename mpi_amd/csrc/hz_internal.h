@@ -194,6 +194,9 @@ int launch_mixed_setup(const MixedSetupArgs &a, hipStream_t s);
 int launch_mixed_modes(const MixedArgs &a, hipStream_t s);
 // Tile rows of the MIXED mode kernel for padded size NP.
 int mixed_tile_rows(int NP);
+// Whether a mode solve of `columns` (kx, ky), N - 2 <= 128, runs mixed_tile's four
+// waves instead of one wave per 16 columns.
+bool mixed_by_four_waves(int n, int ne, int columns);
 
 struct LuFactorArgs {
     double *A;

@@ -79,6 +79,19 @@ int mixed_tile_rows(int NP)
     return (NP == 32 || NP == 96) ? 32 : 16;
 }
 
+// N - 2 padded to 96, several elements and more tiles than two per CU: mixed_tile,
+// whose work-group takes 40 KB of LDS and four waves (four per CU) where six waves
+// with 53 KB are two per CU, and the elements' sweeps, one lane per column, are
+// waited for by fewer others.  Measured, us a solve, mixed_tile | one wave per 16
+// columns: 128^2, Robin, 4 x 67 278 | 284, 6 x 67 467 | 496, periodic 6 x 67
+// 477 | 520; 64^2 periodic 10 x 67 261 | 287, 16 x 67 307 | 347, 16 x 98 339 | 370;
+// below two tiles per CU 32^2 periodic 8 x 67 85 | 76.  (The other padded sizes
+// had 16 rows in mixed_tile and gain everywhere.)
+bool mixed_by_four_waves(int n, int ne, int columns)
+{
+    return diag_padded(n) == 96 && ne >= 4 && columns / (16 / ne) >= 512;
+}
+
 int launch_mixed_setup(const MixedSetupArgs &a, hipStream_t s)
 {
     if (a.modes <= 0) return HZ_OK;
@@ -95,7 +108,8 @@ int launch_mixed_modes(const MixedArgs &a, hipStream_t s)
     switch (diag_padded(a.n)) {
     case 32: return launch_t<2, 32, true>(a, s);
     case 64: return launch_t<4, 32, true>(a, s);
-    case 96: return launch_t<6, 32, true>(a, s);
+    case 96:
+        return mixed_by_four_waves(a.n, a.ne, a.nx * a.M) ? launch_t<6, 32, false>(a, s) : launch_t<6, 32, true>(a, s);
     case 128: return launch_t<8, 32, true>(a, s);
     case 256: return launch_t<16, 16, false>(a, s);
     default: return set_error(HZ_ERR_UNSUPPORTED, "MIXED form: N-2 must be <= 256");

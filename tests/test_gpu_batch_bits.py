@@ -49,7 +49,8 @@ def test_mixed_batch(cuda):
     of faces."""
     sizes = [(5, 1), (18, 8), (34, 3), (35, 1), (66, 2), (67, 5), (98, 1), (99, 4), (130, 1)]
     same_bits([(nx, ny, N, ne, faces) for (nx, ny) in ((32, 16), (1, 32)) for N, ne in sizes
-               for faces in ("dirichlet", "robin", "periodic")], "mixed")
+               for faces in ("dirichlet", "robin", "periodic")]
+              + [(64, 64, 67, 10, "periodic"), (64, 64, 98, 4, "robin")], "mixed")
 
 
 def test_diag_batch_general(cuda):

@@ -203,3 +203,34 @@ def test_plain_panels_of_small_operators_on_many_modes(cuda, N, scale):
     with pytest.raises(HzError):
         plan.status()
     plan.close()
+
+
+@pytest.mark.parametrize("nx,ny,N,ne,periodic", [(32, 32, 67, 9, True), (32, 32, 98, 8, True), (64, 64, 67, 4, False),
+                                                 (64, 64, 98, 3, False), (32, 32, 66, 8, False)])
+def test_mixed_both_kernels_at_the_line_between_them(cuda, nx, ny, N, ne, periodic):
+    """MIXED solves on either side of the rule that sends several elements of 67
+    to 98 points to the four-wave tile: against the oracle within twice its
+    rounding spread (or 1e-12), the residual history falling."""
+    import torch
+    from mpi_amd.solver import HelmholtzPlan
+    from oracle import pyoracle as po
+    lam = 3.0
+    geo = dict(xl=0, xr=2.0, yl=0, yr=3.0, zl=0, zr=2)
+    plan = HelmholtzPlan(nx, ny, N, ne, lam=lam, form="mixed", periodic_z=periodic, **geo)
+    r = np.random.default_rng(N + ne)
+    f = r.standard_normal((nx, ny, plan.nz))
+    g = [r.standard_normal((nx, ny)) for _ in range(2)]
+    dev = lambda v: torch.from_numpy(v).cuda()  # noqa: E731
+    desc = po.make_desc(nx, ny, ne * N, N, size=1, lam=lam, **geo)
+    if periodic:
+        f[:, :, -1] = f[:, :, 0]
+        uo, uf = po.solve_periodic(desc, f), po.solve_periodic(desc, f, fma=True)
+        u = plan.solve(dev(f))
+    else:
+        uo, uf = po.solve(desc, f, *g), po.solve(desc, f, *g, fma=True)
+        u = plan.solve(dev(f), *map(dev, g))
+    bar = max(1e-12, 2.0 * np.abs(uf - uo).max() / np.abs(uo).max())
+    assert np.abs(u.cpu().numpy() - uo).max() <= bar * np.abs(uo).max()
+    h = plan.mixed_history()
+    assert len(h) == 2 and 0 < h[1] < h[0] < 1e-3
+    plan.close()
