@@ -345,7 +345,7 @@ int setup_even_odd(hz_plan *p, const std::vector<double> &A)
         (st = upload(&p->d_eo_B1a, B1a)) || (st = upload(&p->d_eo_B2a, B2a)) || (st = upload(&p->d_eo_M, Mq[0])) ||
         (st = upload(&p->d_eo_Ma, Mq[1])))
         return st;
-    if (zf) {
+    if (zf && !zo.d.empty()) {
         if ((st = upload(&p->d_zf, zo.d)) || (st = upload(&p->d_zf_C, zo.c)) ||
             (st = dmalloc(&p->d_zf_shift, (size_t)p->nx / 2 + 1 + p->M)))
             return st;
@@ -432,10 +432,16 @@ std::array<std::vector<short>, 2> correction_operator(const std::vector<long dou
 // The z-first solve's operands (zfirst.hip) from the even/odd decomposition
 // and M: G_ij = M_ij / (mu_j - mu_i) between the halves, its entries outside
 // the first 16 x 16 block of each half rounded to bf16 as the kernels use
-// them, K = (I - G^2)^-1 (= I + G^2 + G^4 here: G^2 <= 1e-8).  With KW = K
+// them, K = (I - G^2)^-1 (= I + G^2 + G^4 here: G^2 <= 1e-10).  With KW = K
 // Winv: B1 = KW^T, -G; B2 = (D W)^T, +G; face loads K Winv F g, added before the
 // correction.  `d`: B1, B2, X1, X2 (G's FP64 block), w0, wN, then the n
-// eigenvalues, even ones first; `c`: the two bf16 parts.
+// eigenvalues, even ones first; `c`: the two bf16 parts.  Empty if an entry of G
+// is above what the kernels' precisions are meant for: kZfBlock in the FP64 block
+// (first order, G^6 dropped), kZfRest outside it (half a bf16 unit of it is 2e-13
+// of the value).  Of the sizes 3 to 130 the largest are 3.0e-6 (N = 127) and
+// 4.5e-11 (124), whatever Lz.
+constexpr double kZfBlock = 1e-5, kZfRest = 1e-10;
+
 ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::vector<double> &W,
                        const std::vector<double> &Wi, const std::vector<long double> &M,
                        const std::vector<long double> &fg0, const std::vector<long double> &fgN)
@@ -454,6 +460,7 @@ ZfOperands zf_operands(int n, int NP, const std::vector<double> &mu, const std::
             if (!real(i) || !real(j) || (i < H) == (j < H)) continue;
             const double g = (double)(M[(size_t)i * NP + j] / ((long double)mu[j] - (long double)mu[i]));
             const bool block = i % H < 16 && j % H < 16;
+            if (!(std::fabs(g) <= (block ? kZfBlock : kZfRest))) return ZfOperands{};
             at(G, i, j) = block ? g : bf16_value(bf16_of(g));
         }
     auto product = [&](std::vector<double> &out, const std::vector<double> &a, const std::vector<double> &b) {

@@ -37,8 +37,9 @@
 // stay on the z side: V' = V (I + G), G_ij = M_ij / (mu_j - mu_i), and V'^-1 =
 // (I - G) K V^-1 with K = (I - G^2)^-1 (block diagonal, folded into the
 // operand).  The largest eigenvalues come in nearly equal even/odd pairs, so
-// G reaches 1e-6 there (N = 130): its first 16 x 16 block runs in FP64, the
-// rest (below 3e-11) in bf16 with FP32 sums, the values in two parts.
+// G reaches 3e-6 there (N = 127): its first 16 x 16 block runs in FP64, the
+// rest (to 4.5e-11, N = 124) in bf16 with FP32 sums, the values in two parts.
+// A plan whose G is larger keeps transform - mode solve - transform.
 #include "diag_body.h"
 #include "fft_body.h"
 
