@@ -281,9 +281,9 @@ struct hz_plan {
     double Lx = 0, Ly = 0, Lz = 0;
     std::vector<double> z, Dz, Dzz, shift;
     // device
-    double *d_Dz = nullptr, *d_Dzz = nullptr, *d_DzzT = nullptr, *d_offmax = nullptr, *d_shift = nullptr;
-    double *d_DzT = nullptr;  // hz_derivative_z's operands: Dz's, then (DzT_n further on) Dzz's
-    size_t DzT_n = 0;
+    double *d_Dz = nullptr, *d_Dzz = nullptr, *d_DzzT = nullptr, *d_offmax = nullptr;  // one allocation, with ..
+    double *d_DzT[2] = {nullptr, nullptr};  // .. hz_derivative_z's operands of Dz and of Dzz
+    double *d_shift = nullptr;
     double2 *d_twx = nullptr, *d_twy = nullptr;
     hz::Spectrum spec, bc;
     int *d_status = nullptr;

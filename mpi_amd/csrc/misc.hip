@@ -312,5 +312,5 @@ extern "C" int hz_derivative_z(hz_plan *p, int order, const double *u, double *o
 {
     if (!p || !u || !out || (order != 1 && order != 2)) return set_error(HZ_ERR_ARG, "bad argument");
     const long long ncols = (long long)p->ne * p->nx * p->ny;
-    return launch_derivative(order == 1 ? p->d_DzT : p->d_DzT + p->DzT_n, p->N, ncols, u, out, (hipStream_t)stream);
+    return launch_derivative(p->d_DzT[order - 1], p->N, ncols, u, out, (hipStream_t)stream);
 }
