@@ -298,13 +298,19 @@ int hz_mixed_history(const hz_plan *plan, double *rel_residual, int max_sweeps, 
  * none when only one candidate holds the plan), and the
  * z lanes per work-group chosen for each of the four transform passes
  * (R2C y, C2C x, C2C^-1 x, C2R y; 0 = the length's only shape) with the
- * winner's ms.  Any pointer may be NULL.  No counterpart in the reference. */
+ * winner's ms.  The DIAG tile rows are those of the tile kernel: a plan whose
+ * solves go elsewhere (one Dirichlet element through the z-first kernels; N - 2
+ * <= 32 with several elements, Robin faces or periodic z, one wave per 16
+ * columns) is timed and reported all the same, and runs it in its adjoint (the
+ * former) or after hz_plan_set_robin has changed the faces, or not at all.
+ * Any pointer may be NULL.  No counterpart in the reference. */
 int hz_plan_tuning(const hz_plan *plan, int *diag_tile_rows, double *diag_ms, int max_diag,
                    int *fft_lanes, double *fft_ms);
 /* The mode kernel's candidate shapes (DIAG tile rows, or PLAIN_LU column
  * capacities), in the order of hz_plan_tuning's diag_ms (*count = their
  * number, at most `max` written), and a way to pin one of them (a DIAG tile
- * must hold one column's 2*ne element rows).  For tests and tuning studies;
+ * must hold one column's 2*ne element rows).  A pinned tile has no effect on
+ * solves that do not run it (hz_plan_tuning).  For tests and tuning studies;
  * no counterpart in the reference. */
 int hz_plan_diag_candidates(const hz_plan *plan, int *tile_rows, int max, int *count);
 int hz_plan_set_diag_tile(hz_plan *plan, int tile_rows);

@@ -331,7 +331,9 @@ __device__ __forceinline__ int compact(int j, int he, int ho)
 // in 50 us.  The 1,024 work-groups run as two rounds whose loads (16% of a
 // work-group's life), contraction (24%, near the matrix rate of the two that
 // share a CU), correction (20%) and stores hardly overlap: without the loads
-// 41 us, without the contraction 33, without the stores 44.
+// 41 us, without the contraction 33, without the stores 44.  Measured by the
+// counters: 157 MB, matrix cores busy 37% of the SIMD cycles.  Bounded to 128
+// registers it keeps 48 bytes a lane in scratch (16 at smaller NJ).
 template <int NJ, bool CUB>
 __device__ __forceinline__ void expand_tile(const ZfArgs &a, int c0, int tid, EndLds<NJ> &lds)
 {
@@ -396,7 +398,8 @@ __device__ __forceinline__ void expand_tile(const ZfArgs &a, int c0, int tid, En
 }
 
 // ---- 3: 16-point stage back, correction, contraction, store --------------------
-// zf_expand's mirror image and bounds; 256^2 x 129: 56 us.
+// zf_expand's mirror image and bounds; 256^2 x 129: 140 MB in 54 us, matrix cores
+// busy 34% of the SIMD cycles, 16 bytes a lane in scratch.
 template <int NJ>
 __device__ __forceinline__ void collect_tile(const ZfArgs &a, int c0, int tid, EndLds<NJ> &lds)
 {
@@ -518,7 +521,7 @@ __device__ __forceinline__ void end_tiles_of(const ZfArgs &a, int task, char *sm
 // Every problem of a batch in one launch: its tasks of different sizes fill the
 // chip together, where a launch per size leaves most of it idle for the 10 to
 // 20 us that one work-group takes (64 problems, 317 MB: expand 130 us against
-// 147 in four launches, collect 140 against 169).
+// 147 in four launches, collect 140 against 169).  32 bytes a lane in scratch.
 template <bool COLLECT>
 __global__ __launch_bounds__(512, 4) void zf_end_list(const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
 {
@@ -552,7 +555,8 @@ struct Filter {
     static constexpr int NCH = 16 * T / CH;           // blocks per work-group
     static constexpr int LR = R2 + 1;
     // 16-point stages along y in both directions take 162 registers: bounded to
-    // 128 they spill 144 bytes a thread (45 us against 38 at 256^2 x 129)
+    // 128 they spill 144 bytes a thread (45 us against 38 at 256^2 x 129); the
+    // others fit but for 28 bytes of 64 x 128's
     static constexpr int WAVES = R2 == 16 ? 3 : 4;
     static constexpr int LDS = NCH * NX * LR;         // doubles
     static_assert(NCH >= 1, "a block fits a work-group");
@@ -752,7 +756,7 @@ __global__ __launch_bounds__(64, 3) void zf_filter_list64(const ZfArgs *__restri
     }
 }
 
-// A larger grid of a batch.
+// A larger grid of a batch (32 x 256 keeps 48 bytes a lane in scratch).
 template <int NX, int R2>
 __global__ __launch_bounds__((Filter<NX, R2>::T), (Filter<NX, R2>::WAVES)) void zf_filter_list(
     const ZfArgs *__restrict__ Z, const int2 *__restrict__ list)
@@ -816,11 +820,13 @@ int launch_filter(const ZfArgs &a, hipStream_t s)
 // Three launches instead of five, but few work-groups on a small grid: an end
 // kernel has nx ny / 64, each 10 to 16 us from its first load to its last store
 // (N = 130), against the transform passes' many short ones.  Measured, us a
-// solve, here against transform - mode solve - transform: 64 x 64 x 130 38.4 |
-// 34.7, 32 x 256 x 130 53.3 | 49.1; 128 x 64 x 18 24.0 | 23.1, x 66 29.8 | 31.0,
-// x 130 45.2 | 49.3; 64 x 256 x 18 26.8 | 27.3, x 130 55.2 | 66.9; 256^2 x 3 28.9 |
-// 33.9, x 130 132 | 165.  N - 2 > 128 would need a larger FP64 block of the
-// correction and a 512-point axis blocks of the filter beyond the registers.
+// solve, here against transform - mode solve - transform: 64 x 64 x 130 38.5 |
+// 33.8, 32 x 256 x 130 49.2 | 47.6; 128 x 64 x 18 21.7 | 20.9, x 66 29.8 | 30.7,
+// x 130 45.7 | 47.9; 64 x 128 x 66 32.0 | 30.5, x 99 44.2 | 42.6, x 130 47.7 |
+// 48.2; 64 x 256 x 18 23.3 | 25.0, x 130 50.7 | 65.0; 256^2 x 3 26.6 | 32.9, x 67
+// 112 | 108, x 98 128 | 131, x 130 135 | 164.  N - 2 > 128 would need end kernels
+// of 256 eigen-indices and a larger FP64 block of the correction, a 512-point
+// axis filter blocks of 1,024 threads and 135 KB of LDS (512 x 32 points).
 bool zf_holds(int nx, int ny, int n)
 {
     if (nx < 64 || nx > 256 || ny < 32 || ny > 256 || n < 1 || n > 128) return false;
