@@ -833,7 +833,7 @@ static bool stepwise(int n, int c, int modes)
         int n, c;
         long long work, work4;
     } lines[] = {{1, 30, 68000, 1LL << 62}, {2, 30, 24000, 1LL << 62}, {3, 30, 14000, 48000}, {4, 28, 9200, 22000},
-                 {5, 28, 6800, 6800},       {6, 24, 4800, 4800},       {7, 20, 4400, 4400},   {8, 16, 2400, 2400},
+                 {5, 28, 6800, 6800},       {6, 24, 4800, 4800},       {7, 20, 4400, 4400},   {8, 16, 2400, 2800},
                  {10, 10, 1200, 1200},      {12, 6, 400, 400},         {14, 4, 140, 140},     {16, 0, 0, 0},
                  {18, 10, 1200, 1200},      {20, 6, 480, 480},         {22, 6, 400, 400},     {26, 4, 140, 140},
                  {32, 0, 0, 0},             {35, 4, 140, 140}};
