@@ -116,7 +116,7 @@ def test_derivative_z_few_and_many_outputs(cuda, nx, ny, N):
 @pytest.mark.parametrize("N", [3, 4])
 def test_plain_smallest_operators_are_short(cuda, N):
     """The reference algorithm with one or two interior nodes against seven: at
-    most three quarters of the time (16-column panels cost nearly the same)."""
+    most four fifths of the time (16-column panels cost nearly the same)."""
     import torch
     from mpi_amd.solver import HelmholtzPlan
     took = []
@@ -127,7 +127,7 @@ def test_plain_smallest_operators_are_short(cuda, N):
         u = plan.empty_field()
         took.append(best_us(lambda: plan.solve(f, g, g, out=u)))
         plan.close()
-    assert took[0] <= 0.75 * took[1], took
+    assert took[0] <= 0.8 * took[1], took
 
 
 @pytest.mark.parametrize("nx,ny,N,ne", [(1, 1, 3, 1), (256, 64, 3, 4), (128, 128, 4, 1), (128, 128, 4, 2),
